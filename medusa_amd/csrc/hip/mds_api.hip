@@ -21,7 +21,7 @@ extern "C" hipError_t mds_launch_sweep1d(int fp32, int nv, int sph, int tab, int
                                          const void *sp, const void *sph_, int stage, hipStream_t st);
 extern "C" hipError_t mds_launch_slab_fill(int fp32, const DevProb *probs, int nprob, long long items,
                                            void *const *state, const DevEos *eos, int tab, int nv, hipStream_t st);
-extern "C" hipError_t mds_launch_monopole(int fp32, int mono, int tab, int nprob, const DevProb *prob,
+extern "C" hipError_t mds_launch_monopole(int fp32, int mono, int tab, int nprob, int nmax, const DevProb *prob,
                                           const DevClock *clock, const DevEos *eos, const void *st, double *grav,
                                           hipStream_t s);
 hipError_t mds_eos_to_device(const mds_eos_table *t, DevEos *d, void **alloc);
@@ -68,6 +68,7 @@ struct mds_ctx {
   int nseg2 = 0;
   int2 *dseg3 = nullptr;           // the same for two zones per lane (FP32-bulk)
   int nseg3 = 0;
+  int nmax1d = 0;                  // 1D: zones of the largest column
   int can_fuse1d = 0;              // 1D and no problem periodic in x
   int fuse1d = 0;                  // use the two-stage 1D kernel (p -> ph, then swap); 2: two zones per lane
   int par = 0;                     // buffer parity: which allocation p currently names
@@ -875,6 +876,7 @@ static int create_impl(mds_ctx *c, const mds_problem *probs, int nprob, const md
     HIPCHK(c, hipMemcpy(c->dseg3, seg.data(), sizeof(int2) * seg.size(), hipMemcpyHostToDevice));
     // the two-stage kernel needs every ghost source zone inside the wave, and
     // no field that depends on the whole column between the stages
+    for (const DevProb &h : c->hprob) c->nmax1d = std::max(c->nmax1d, h.n[0]);
     c->can_fuse1d = !c->mono && !c->has_slab && rp->hydro_interp_order == 3;
     for (int p = 0; p < nprob; p++)
       if (c->hprob[p].bc_lo[0] == MDS_BC_PERIODIC || c->hprob[p].bc_hi[0] == MDS_BC_PERIODIC) c->can_fuse1d = 0;
@@ -1109,13 +1111,13 @@ static int enqueue_stage(mds_ctx *c, int stage, int fp32)
       StateArrays<float> sp = arrays<float>(c->p), sh = arrays<float>(c->ph);
       // monopole field of the stage input state (gravity.c:145-251 at p_to_phys_src_start)
       if (c->mono)
-        HIPCHK(c, mds_launch_monopole(1, c->mono, c->tab, c->nprob, c->dprob, c->dclock, &c->deos,
+        HIPCHK(c, mds_launch_monopole(1, c->mono, c->tab, c->nprob, c->nmax1d, c->dprob, c->dclock, &c->deos,
                                       stage == 0 ? &sp : &sh, c->dgrav, c->st));
       HIPCHK(c, mds_launch_sweep1d(1, c->nv, c->sph, c->tab, c->mono, &a, &sp, &sh, stage, c->st));
     } else {
       StateArrays<double> sp = arrays<double>(c->p), sh = arrays<double>(c->ph);
       if (c->mono)
-        HIPCHK(c, mds_launch_monopole(0, c->mono, c->tab, c->nprob, c->dprob, c->dclock, &c->deos,
+        HIPCHK(c, mds_launch_monopole(0, c->mono, c->tab, c->nprob, c->nmax1d, c->dprob, c->dclock, &c->deos,
                                       stage == 0 ? &sp : &sh, c->dgrav, c->st));
       HIPCHK(c, mds_launch_sweep1d(0, c->nv, c->sph, c->tab, c->mono, &a, &sp, &sh, stage, c->st));
     }

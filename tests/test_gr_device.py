@@ -212,3 +212,25 @@ def test_gr_star3d_matches_oracle(dendritic, use_table, precision):
     for k, v in err.items():
         assert v <= tol, (k, v)
     _gr_state_close(ctx.gr_state(), sim, 1e-12 if precision == 0 else 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n, rho_c", [(12, 1.0e10), (256, 1.0e10), (257, 1.0e14), (1024, 1.0e14), (1025, 1.0e10)])
+def test_gr_faces_at_the_edges_of_the_tiles_match_oracle(n, rho_c):
+    """The face recurrence is solved a tile of 256 or 1024 faces at a time:
+    columns of fewer faces than a tile, of exactly one and of one more, weak
+    and (rho_c = 1e14, GM / R c^2 some 0.03) stronger fields.  The sums are
+    trees of at most 1025 terms of one sign (errors below 20 eps) and the
+    rounds stop within 2 eps, so five steps stay far within 1e-12."""
+    g, prob, prims = problems.star1d(n, table=None, sigma=0.01, rho_c=rho_c)
+    prob = dict(prob, monopole=mds.MONOPOLE_GR)
+    print(f"[gr] GR star column n={n} rho_c={rho_c:g}, 5 steps", flush=True)
+    ctx = _ctx([prob], mds.FP64, [prims], 5, graph=False)
+    sim = _oracle(prob, None)
+    sim.set_prims(prims)
+    sim.run(max_steps=5)
+    dev, ref = ctx.download(), sim.get_prims()
+    w = g.zone()[2:-2, mds.ZG_VOLUME]
+    assert _rel(dev[0].ravel(), ref[0].ravel(), w) <= FP64_TOL
+    assert _rel(dev[1].ravel(), ref[1].ravel(), w) <= FP64_TOL
+    assert ctx.gr_state()["passes"] == _gr_state_close(ctx.gr_state(), sim, 1e-12)
