@@ -692,6 +692,27 @@ static int create_impl(mds_ctx *c, const mds_problem *probs, int nprob, const md
       if (rc1) return rc1;
       rc1 = upload_geo(c, rcf.data(), rcf.size() * sizeof(float), (const void **)&d.rc[k]);
       if (rc1) return rc1;
+      if (c->precision != MDS_FP32_BULK && g->geom == MDS_GEOM_CARTESIAN && g->ndim > 1) {
+        // the quotients of recon_geo_x64 and the faces of the zones that have
+        // both neighbours
+        std::vector<double> rg((size_t)nzk * MDS_RG_COUNT, 0.0);
+        for (int q = 1; q < nzk - 1; q++) {
+          const double *al = g->alpha[k] + q, *be = g->beta[k] + q, *ga = g->Gamma[k] + q;
+          if (ga[-1] != g->dx[k] || ga[0] != g->dx[k] || ga[1] != g->dx[k])
+            return set_err(c, MDS_EINVAL, "a Cartesian grid's Gamma moments are its zone width");
+          ReconGeo64 z;
+          z.am = al[-1]; z.bm = be[-1]; z.gm = ga[-1];
+          z.a0 = al[0];  z.b0 = be[0];  z.g0 = ga[0];
+          z.ap = al[1];  z.bp = be[1];  z.gp = ga[1];
+          z.xlo = g->startx[k] + (q - MDS_NG) * g->dx[k];
+          z.xhi = g->startx[k] + (q - MDS_NG + 1) * g->dx[k];
+          recon_geo_x64(z);
+          double *o = &rg[(size_t)q * MDS_RG_COUNT];
+          o[MDS_RG_DEN] = z.den; o[MDS_RG_DEN2] = z.den2; o[MDS_RG_XLO] = z.xlo; o[MDS_RG_XHI] = z.xhi;
+        }
+        rc1 = upload_geo(c, rg.data(), rg.size() * sizeof(double), (const void **)&d.rg64[k]);
+        if (rc1) return rc1;
+      }
     }
     if (g->dendritic) {
       // level tables (log2 of dj, dk) and the theta / phi moments of every level

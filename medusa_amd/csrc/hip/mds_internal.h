@@ -41,6 +41,11 @@ enum {
   MDS_TC_C022, MDS_TC_C122, MDS_TC_C220, MDS_TC_C221, MDS_TC_COUNT
 };
 
+// DevProb::rg64: the parts of a zone's FP64 reconstruction geometry that its
+// moments alone fix (recon_geo_x64), made once on the host with the same
+// operations, and its faces
+enum { MDS_RG_DEN = 0, MDS_RG_DEN2, MDS_RG_XLO, MDS_RG_XHI, MDS_RG_COUNT };
+
 struct DevProb {
   long long off;           // first interior zone in the packed state arrays
   int n[3];                // interior zones
@@ -67,6 +72,7 @@ struct DevProb {
   int tcu;
   double tcu_c[MDS_TC_COUNT];
   const double *mom[3];    // per direction (n[d]+2NG)*3: alpha, beta, Gamma per zone
+  const double *rg64[3];   // Cartesian 2D/3D, FP64: per direction (n[d]+2NG)*MDS_RG_COUNT
   const float *rc[3];      // per direction (n[d]+2NG)*MDS_RC_COUNT
   const double *zone;      // spherical columns: (n[0]+2NG) x MDS_ZG_COUNT records; 3D spherical:
                            // field-major, zone[field][j + NG][i + NG] (MDS_ZS_*)

@@ -74,7 +74,7 @@ struct ReconGeo64 {
   int order = 3;         // hydro_interp_order: 3 para_recon, 2 lin_recon, 1 piecewise constant
 };
 
-MDS_DEV void recon_geo_x64(ReconGeo64 &g)
+__host__ MDS_DEV void recon_geo_x64(ReconGeo64 &g)
 {
   double t012 = (g.am * g.b0) * g.gp;
   double t021 = (g.am * g.bp) * g.g0;

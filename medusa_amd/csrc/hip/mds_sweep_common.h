@@ -49,28 +49,60 @@ MDS_DEV void recon(R qm, R q0, R qp, const typename ReconGeoT<R>::type &g, R &al
   else para_recon_f32(qm, q0, qp, g, al, ar);
 }
 
-// reconstruction geometry of zone z (index without ghost offset) in direction d
+// The tables of one direction's reconstruction geometry, read from the problem
+// record once: the record is global memory, and after a march's stores the
+// compiler would read the pointers again before every row's table entries.
 template <class R>
-MDS_DEV void load_rgeo(const DevProb &pb, int d, int z, typename ReconGeoT<R>::type &g)
+struct GeoDir {
+  const double *mom, *rg;
+  const float *rc;
+  double dx;
+  int qmax, order;
+  MDS_DEV GeoDir(const DevProb &pb, int d)
+  {
+    mom = pb.mom[d];
+    rg = pb.rg64[d];
+    rc = pb.rc[d];
+    dx = pb.dx[d];
+    qmax = pb.n[d] + 2 * MDS_NG - 2;
+    order = pb.order;
+  }
+};
+
+// reconstruction geometry of zone z (index without ghost offset)
+template <class R>
+MDS_DEV void load_rgeo(const GeoDir<R> &G, int z, typename ReconGeoT<R>::type &g)
 {
-  int nz = pb.n[d] + 2 * MDS_NG;
   int q = z + MDS_NG;
-  q = q < 1 ? 1 : (q > nz - 2 ? nz - 2 : q);
+  q = q < 1 ? 1 : (q > G.qmax ? G.qmax : q);
   if constexpr (std::is_same<R, double>::value) {
-    const double *m = pb.mom[d];
-    g.am = m[3 * (q - 1) + 0]; g.bm = m[3 * (q - 1) + 1]; g.gm = m[3 * (q - 1) + 2];
-    g.a0 = m[3 * q + 0];       g.b0 = m[3 * q + 1];       g.g0 = m[3 * q + 2];
-    g.ap = m[3 * (q + 1) + 0]; g.bp = m[3 * (q + 1) + 1]; g.gp = m[3 * (q + 1) + 2];
-    g.xlo = pb.startx[d] + z * pb.dx[d];
-    g.xhi = pb.startx[d] + (z + 1) * pb.dx[d];
-    recon_geo_x64(g);
-    g.order = pb.order;
+    // moments of zones q - 1 .. q + 1 and the zone's quotients and faces from
+    // the tables; on Cartesian grids Gamma is dx in every zone
+    const double *m = G.mom + 3 * (q - 1);
+    const double *t = G.rg + (size_t)q * MDS_RG_COUNT;
+    g.am = m[0]; g.bm = m[1];
+    g.a0 = m[3]; g.b0 = m[4];
+    g.ap = m[6]; g.bp = m[7];
+    g.gm = g.g0 = g.gp = G.dx;
+    g.den = t[MDS_RG_DEN]; g.den2 = t[MDS_RG_DEN2];
+    g.xlo = t[MDS_RG_XLO]; g.xhi = t[MDS_RG_XHI];
+    g.order = G.order;
   } else {
-    const float *r = pb.rc[d] + (size_t)q * MDS_RC_COUNT;
+    const float *r = G.rc + (size_t)q * MDS_RC_COUNT;
     g.clm = r[MDS_RC_CLM]; g.clp = r[MDS_RC_CLP]; g.crm = r[MDS_RC_CRM]; g.crp = r[MDS_RC_CRP];
     g.mu1 = r[MDS_RC_MU1]; g.kinv = r[MDS_RC_KINV]; g.inur = r[MDS_RC_INUR]; g.imu2 = r[MDS_RC_IMU2];
   }
 }
+
+// Keeps the expressions of a zone's geometry (xlo xlo, xlo - xhi, the A3
+// denominators ...) out of loop-invariant registers: the x geometry of a lane
+// is fixed over a march, and hoisting them would hold some ten more doubles
+// per lane through it than the zone data leave room for.
+MDS_DEV void pin_rgeo(ReconGeo64 &g)
+{
+  asm volatile("" : "+v"(g.xlo), "+v"(g.xhi), "+v"(g.a0), "+v"(g.b0));
+}
+MDS_DEV void pin_rgeo(ReconGeo32 &) {}
 
 // A stencil zone in a ghost layer of a PROB or EXTRAP side: its entries
 // (entry v at e[v * T]).  The first such direction decides; the transverse
@@ -118,6 +150,34 @@ MDS_DEV void load_cell(const StateArrays<R> &in, const DevProb &pb, int i, int j
   c.rho = in.v[0][idx];
   c.uu = in.v[1][idx];
   for (int d = 0; d < NV; d++) c.v[d] = in.v[2 + d][idx];
+  if (fx) c.v[0] = -c.v[0];
+  if (fy && NV > 1) c.v[1] = -c.v[1];
+  if (fz && NV > 2) c.v[2] = -c.v[2];
+  c.P = gm1 * c.uu;
+}
+
+// Entry idx of the row that starts at zone rb.  The row (its number, mapping
+// and flips) is uniform over the wavefront and stays in scalar registers:
+// every access is the scalar address of its array's row plus the lane's byte
+// offset, so a row costs no vector address arithmetic.
+template <class T>
+MDS_DEV T ld_row(const T *base, long long rb, int idx)
+{
+  return *(const T *)((const char *)(base + rb) + (unsigned)idx * (unsigned)sizeof(T));
+}
+template <class T>
+MDS_DEV void st_row(T *base, long long rb, int idx, T v)
+{
+  *(T *)((char *)(base + rb) + (unsigned)idx * (unsigned)sizeof(T)) = v;
+}
+
+template <class R, int NV>
+MDS_DEV void load_row_cell(const StateArrays<R> &in, long long rb, int si, bool fx, bool fy, bool fz, R gm1,
+                           Cell<R, NV> &c)
+{
+  c.rho = ld_row(in.v[0], rb, si);
+  c.uu = ld_row(in.v[1], rb, si);
+  for (int d = 0; d < NV; d++) c.v[d] = ld_row(in.v[2 + d], rb, si);
   if (fx) c.v[0] = -c.v[0];
   if (fy && NV > 1) c.v[1] = -c.v[1];
   if (fz && NV > 2) c.v[2] = -c.v[2];
