@@ -418,43 +418,48 @@ MDS_DEV float frsqrt(float x) { return __builtin_amdgcn_rsqf(x); }
 // a few 1e-7 for |y log2 x| near 10, within what FP32 storage already makes
 MDS_DEV float fpow(float x, float y) { return __builtin_amdgcn_exp2f(y * __builtin_amdgcn_logf(x)); }
 
-// para_recon in local coordinates: identical branch structure, well-conditioned.
+// para_recon in local coordinates: the same limiter, on the face values'
+// offsets L, R from the zone mean.  With the parabola's slopes d0 = b1 and
+// d1 = b1 + 2 b2 at the faces and D = R - L at the middle, its extremum lies
+// inside the zone where d0 d1 < 0, in the upper half where d0 D > 0: no
+// reciprocal, and 34 instructions against the 45 slots of the form that
+// located it.  The FP32 kernels are bound by vector issue: with the shorter
+// star pressure and star flux below, KH 2048^2 went from 282 to 248 us a step,
+// RT 256^3 from 2.28 to 1.98 ms.  Against 64-bit runs the errors are what they
+// were (KH 1.09e-7 -> 1.06e-7, tubes 1.31e-7 -> 1.23e-7, all variables).
 MDS_DEV void para_recon_f32(float qm, float q0, float qp, const ReconGeo32 &g, float &al, float &ar)
 {
 #pragma clang fp contract(fast)
-  float dqm = q0 - qm;
-  float dqp = qp - q0;
+  const float dqm = q0 - qm;
+  const float dqp = qp - q0;
+  // a local extremum or a uniform stretch, where whole wavefronts skip the rest
   if (dqm * dqp <= 0.0f) { al = q0; ar = q0; return; }
-  float l = q0 + g.clm * dqm + g.clp * dqp;
-  float r = q0 + g.crm * dqm + g.crp * dqp;
-  float mean = 0.75f * qm + 0.25f * q0;
-  if ((q0 - l) * (l - mean) < 0.0f) l = mean;
-  mean = 0.75f * qp + 0.25f * q0;
-  if ((mean - r) * (r - q0) < 0.0f) r = mean;
-  float b2 = (q0 - l - (r - l) * g.mu1) * g.kinv;
-  float b1 = (r - l) - b2;
-  // extremum sigma* = -b1/(2 b2) strictly inside (0,1)?
-  float sz = -b1 * frcp(2.0f * b2);
-  if (b2 != 0.0f && sz > 0.0f && sz < 1.0f) {
-    if (sz > 0.5f) l = r + (q0 - r) * g.inur;
-    else r = l + (q0 - l) * g.imu2;
-  }
-  al = l;
-  ar = r;
+  float L = g.clm * dqm + g.clp * dqp;
+  float R = g.crm * dqm + g.crp * dqp;
+  // outside the span of the zone mean and 3/4 of the step to the neighbour
+  if (L * (L + 0.75f * dqm) > 0.0f) L = -0.75f * dqm;
+  if (R * (R - 0.75f * dqp) > 0.0f) R = 0.75f * dqp;
+  const float D = R - L;
+  const float b2 = (-L - D * g.mu1) * g.kinv;
+  const float d0 = D - b2, d1 = D + b2;
+  const bool in = d0 * d1 < 0.0f, up = d0 * D > 0.0f;
+  const float Ln = R - R * g.inur, Rn = L - L * g.imu2;
+  if (in && up) L = Ln;
+  if (in && !up) R = Rn;
+  al = q0 + L;
+  ar = q0 + R;
 }
 
-// Gamma-only factors of the FP32 wave-speed estimate, each formed exactly as
-// wave_speeds_f32 forms it from a side's Gamma_1 (with G_l = G_r = G, G_avg
-// is G itself).  A gamma law needs one set per launch: gam_f32_uniform makes
-// it once and keeps it in scalar registers, and the shock and rarefaction
-// branches then take no reciprocal of Gamma per face.
+// Gamma-only factors of the FP32 wave-speed estimate.  A gamma law needs one
+// set per launch: gam_f32_uniform makes it once and keeps it in scalar
+// registers, and the shock and rarefaction branches then take no reciprocal
+// of Gamma per face.
 struct GamF32 {
   float ravg;  // (G - 1) rcp(2 G): exponent of the two-rarefaction pressure ratio
-  float igm1;  // rcp(G - 1)
   float hgm1;  // (G - 1) / 2
   float pex;   // 2 G rcp(G - 1): power of the two-rarefaction star pressure
-  float gp1;   // G + 1
   float bgm;   // (G - 1) rcp(G + 1): the two-shock b / p
+  float sgp1;  // sqrt((G + 1) / 2): the two-shock velocity scale
   float kq;    // (G + 1) rcp(2 G): the shock factor's slope
 };
 MDS_DEV float uniform_f32(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
@@ -462,11 +467,10 @@ MDS_DEV GamF32 gam_f32_uniform(float G)
 {
   GamF32 k;
   k.ravg = uniform_f32((G - 1.0f) * frcp(2.0f * G));
-  k.igm1 = uniform_f32(frcp(G - 1.0f));
   k.hgm1 = uniform_f32((G - 1.0f) * 0.5f);
   k.pex = uniform_f32(2.0f * G * frcp(G - 1.0f));
-  k.gp1 = uniform_f32(G + 1.0f);
   k.bgm = uniform_f32((G - 1.0f) * frcp(G + 1.0f));
+  k.sgp1 = uniform_f32(fsqrt(0.5f * (G + 1.0f)));
   k.kq = uniform_f32((G + 1.0f) * frcp(2.0f * G));
   return k;
 }
@@ -484,83 +488,80 @@ MDS_DEV GamSet gam_set_uniform(double G)
   return k;
 }
 
-// EAGER: both pressure reciprocals up front, serving the ratio and both
-// shock factors (faster where shock factors are common, as on Cartesian
+// EAGER: both pressure reciprocals up front, serving the rarefactions and
+// both shock factors (faster where shock factors are common, as on Cartesian
 // boxes); otherwise the shock factors divide only where a wavefront needs them.
-// UNIG: G_l = G_r, with its factors in *gk (a gamma law).
-template <bool HLLC_FLOOR, bool EAGER = false, bool UNIG = false>
+// UNIG: G_l = G_r, with its factors in *gk (a gamma law).  rs_l, rs_r:
+// rsqrt(rho), which the sound speeds have formed already.
+template <bool EAGER = false, bool UNIG = false>
 MDS_DEV void wave_speeds_f32(float rl, float rr, float p_l, float p_r, float G_l, float G_r,
-                             float u_l, float u_r, float cs_l, float cs_r,
+                             float u_l, float u_r, float cs_l, float cs_r, float rs_l, float rs_r,
                              float &sl, float &sr, float &ss, float &p_s, int &isshock,
                              const GamF32 *gk = nullptr)
 {
 #pragma clang fp contract(fast)
-  float p_max = fmaxf(p_l, p_r), p_min = fminf(p_l, p_r);
-  float ipl = 0.0f, ipr = 0.0f, ipmin;
+  const float p_max = fmaxf(p_l, p_r), p_min = fminf(p_l, p_r);
+  const float du = u_r - u_l;
+  float ipl = 0.0f, ipr = 0.0f;
   if constexpr (EAGER) {
     ipl = frcp(p_l);
     ipr = frcp(p_r);
-    ipmin = p_l <= p_r ? ipl : ipr;
-  } else {
-    ipmin = frcp(p_min);
   }
-  float pratio = p_max * ipmin;
-  isshock = ((p_max - p_min) * ipmin > 0.5f) ? 1 : 0;
-  p_s = 0.5f * (p_l + p_r) - 0.125f * (u_r - u_l) * (rl + rr) * (cs_l + cs_r);
+  isshock = (p_max - p_min > 0.5f * p_min) ? 1 : 0;
+  p_s = 0.5f * (p_l + p_r) - 0.125f * du * (rl + rr) * (cs_l + cs_r);
   p_s = fmaxf(p_s, 0.0f);
-  if (pratio < 2.0f && p_s >= p_min && p_s <= p_max) {
+  if (p_max < 2.0f * p_min && p_s >= p_min && p_s <= p_max) {
   } else if (p_s < p_min) {
-    float G_avg = 0.5f * (G_l + G_r);
-    const float ex = UNIG ? gk->ravg : (G_avg - 1.0f) * frcp(2.0f * G_avg);
-    float plr = fpow(p_l * (EAGER ? ipr : frcp(p_r)), ex);
-    float icl = frcp(cs_l), icr = frcp(cs_r);
-    const float igm1 = UNIG ? gk->igm1 : frcp(G_avg - 1.0f);
-    float s0 = (plr * u_l * icl + u_r * icr + 2.0f * (plr - 1.0f) * igm1) * frcp(plr * icl + icr);
-    const float hl = UNIG ? gk->hgm1 : (G_l - 1.0f) * 0.5f, hr = UNIG ? gk->hgm1 : (G_r - 1.0f) * 0.5f;
-    const float el = UNIG ? gk->pex : 2.0f * G_l * frcp(G_l - 1.0f);
-    const float er = UNIG ? gk->pex : 2.0f * G_r * frcp(G_r - 1.0f);
-    p_s = 0.5f * (p_l * fpow(1.0f + hl * icl * (u_l - s0), el) + p_r * fpow(1.0f + hr * icr * (s0 - u_r), er));
+    const float plr = fpow(p_l * (EAGER ? ipr : frcp(p_r)),
+                           UNIG ? gk->ravg : (0.5f * (G_l + G_r) - 1.0f) * frcp(G_l + G_r));
+    if constexpr (UNIG) {
+      // both sides' star pressures in one: with one Gamma the left and the
+      // right isentrope meet at p_l [(c_l + c_r - h du) / (c_l + c_r plr)]^pex,
+      // which is what their mean is; the bracket as one less its distance
+      // from one, which the power would multiply the rounding of
+      p_s = p_l * fpow(1.0f - (gk->hgm1 * du + cs_r * (plr - 1.0f)) * frcp(cs_l + cs_r * plr), gk->pex);
+    } else {
+      const float icl = frcp(cs_l), icr = frcp(cs_r);
+      const float igm1 = frcp(0.5f * (G_l + G_r) - 1.0f);
+      const float s0 = (plr * u_l * icl + u_r * icr + 2.0f * (plr - 1.0f) * igm1) * frcp(plr * icl + icr);
+      const float hl = (G_l - 1.0f) * 0.5f, hr = (G_r - 1.0f) * 0.5f;
+      const float el = 2.0f * G_l * frcp(G_l - 1.0f), er = 2.0f * G_r * frcp(G_r - 1.0f);
+      p_s = 0.5f * (p_l * fpow(1.0f + hl * icl * (u_l - s0), el) + p_r * fpow(1.0f + hr * icr * (s0 - u_r), er));
+    }
     p_s = fmaxf(p_s, 0.0f);
   } else {
-    float a_l = 2.0f * frcp((UNIG ? gk->gp1 : G_l + 1.0f) * rl);
-    float a_r = 2.0f * frcp((UNIG ? gk->gp1 : G_r + 1.0f) * rr);
-    float b_l = (UNIG ? gk->bgm : (G_l - 1.0f) * frcp(G_l + 1.0f)) * p_l;
-    float b_r = (UNIG ? gk->bgm : (G_r - 1.0f) * frcp(G_r + 1.0f)) * p_r;
-    // sqrt(a / (p + b)) as sqrt(a) / sqrt(p + b): the quotient itself falls
-    // below the FP32 normal range at stellar-core densities and pressures
-    // (2 / (2.3 rho) / (p + b) near 1e-38 at rho 1e10, p 1e28), where the
-    // hardware square root flushes it to zero
-    float g_l = fsqrt(a_l) * frsqrt(p_s + b_l);
-    float g_r = fsqrt(a_r) * frsqrt(p_s + b_r);
-    p_s = (g_l * p_l + g_r * p_r - (u_r - u_l)) * frcp(g_l + g_r);
+    // the two-shock weights sqrt(2 / ((G + 1) rho) / (p_s + b)) as products of
+    // reciprocal roots: the quotient itself falls below the FP32 normal range
+    // at stellar-core densities and pressures, where the hardware roots flush
+    // it to zero.  With one Gamma their common sqrt(2 / (G + 1)) moves to du.
+    const float b_l = (UNIG ? gk->bgm : (G_l - 1.0f) * frcp(G_l + 1.0f)) * p_l;
+    const float b_r = (UNIG ? gk->bgm : (G_r - 1.0f) * frcp(G_r + 1.0f)) * p_r;
+    float g_l = rs_l * frsqrt(p_s + b_l);
+    float g_r = rs_r * frsqrt(p_s + b_r);
+    float dv = du;
+    if constexpr (UNIG) {
+      dv = du * gk->sgp1;
+    } else {
+      g_l *= frsqrt(0.5f * (G_l + 1.0f));
+      g_r *= frsqrt(0.5f * (G_r + 1.0f));
+    }
+    p_s = (g_l * p_l + g_r * p_r - dv) * frcp(g_l + g_r);
     p_s = fmaxf(p_s, 0.0f);
   }
   const float kl = UNIG ? gk->kq : (G_l + 1.0f) * frcp(2.0f * G_l);
   const float kr = UNIG ? gk->kq : (G_r + 1.0f) * frcp(2.0f * G_r);
   float q_l = (p_s <= p_l) ? 1.0f : fsqrt(1.0f + kl * (p_s * (EAGER ? ipl : frcp(p_l)) - 1.0f));
   float q_r = (p_s <= p_r) ? 1.0f : fsqrt(1.0f + kr * (p_s * (EAGER ? ipr : frcp(p_r)) - 1.0f));
-  sl = u_l - cs_l * q_l;
-  sr = u_r + cs_r * q_r;
-  ss = (p_r - p_l + rl * u_l * (sl - u_l) - rr * u_r * (sr - u_r)) * frcp(rl * (sl - u_l) - rr * (sr - u_r));
+  // the waves' speeds against the gas and the mass fluxes through them
+  const float w_l = cs_l * q_l, w_r = cs_r * q_r;
+  const float m_l = rl * w_l, m_r = rr * w_r;
+  sl = u_l - w_l;
+  sr = u_r + w_r;
+  ss = (p_l - p_r + u_l * m_l + u_r * m_r) * frcp(m_l + m_r);
 }
 
-// Per-unit-area fluxes in FP32 (the FP64 caller applies the FP64 area).
-template <int NV, bool CART, int NS = 0>
-MDS_DEV void pflux_f32(const PState<float, NV> &p, const FaceGeo<float> &g, int dir, float f[6])
-{
-#pragma clang fp contract(fast)
-  float vcov[3];
-  for (int d = 0; d < NV; d++) vcov[d] = CART ? p.v[d] : g.gcov[d] * p.v[d];
-  float v = p.v[dir];
-  f[0] = p.rho * v;
-  for (int d = 0; d < NV; d++) f[2 + d] = f[0] * vcov[d];
-  f[2 + dir] += p.P;
-  float vsq = 0.0f;
-  for (int d = 0; d < NV; d++) vsq += p.v[d] * vcov[d];
-  f[1] = v * (0.5f * p.rho * vsq + p.uu + p.P);
-  if (NS) f[MDS_YI] = f[0] * p.ye;
-}
-
+// Conserved state and per-unit-area physical flux of one side in FP32 (the
+// FP64 caller applies the FP64 area).
 template <int NV, bool CART, int NS = 0>
 MDS_DEV void p_uflux_f32(const PState<float, NV> &p, const FaceGeo<float> &g, int dir, float u[6], float f[6])
 {
@@ -590,12 +591,13 @@ MDS_DEV int hllc_f32(const PState<float, NV> &L, const PState<float, NV> &Rt,
 #pragma clang fp contract(fast)
   float u_l = CART ? L.v[dir] : L.v[dir] * g.scale;
   float u_r = CART ? Rt.v[dir] : Rt.v[dir] * g.scale;
-  float cs_l = fsqrt(L.G * L.P * frcp(L.rho));
-  float cs_r = fsqrt(Rt.G * Rt.P * frcp(Rt.rho));
+  const float rs_l = frsqrt(L.rho), rs_r = frsqrt(Rt.rho);
+  float cs_l = fsqrt(L.G * L.P) * rs_l;
+  float cs_r = fsqrt(Rt.G * Rt.P) * rs_r;
   float sl, sr, ss, p_s;
   int isshock;
-  wave_speeds_f32<true, CART, UNIG>(L.rho, Rt.rho, L.P, Rt.P, L.G, Rt.G, u_l, u_r, cs_l, cs_r, sl, sr, ss, p_s,
-                                    isshock, gk);
+  wave_speeds_f32<CART, UNIG>(L.rho, Rt.rho, L.P, Rt.P, L.G, Rt.G, u_l, u_r, cs_l, cs_r, rs_l, rs_r, sl, sr, ss, p_s,
+                              isshock, gk);
   if (ss > sr) sr = 1.001f * ss;
   if (ss < sl) sl = 1.001f * ss;
   float iscale = CART ? 1.0f : frcp(g.scale);
@@ -605,22 +607,29 @@ MDS_DEV int hllc_f32(const PState<float, NV> &L, const PState<float, NV> &Rt,
   // else the side of the contact), plus the star-state term where neither
   // wave is supersonic (riemann.c:437-495).  The term is selected, not
   // weighted, so an undefined star state of a supersonic face stays out.
+  // The transverse velocities (and Ye) do not change across the waves, so
+  // their fluxes are the mass flux times the upwind value.
   const bool sup_l = sl > 0.0f, sup_r = sr < 0.0f, star = !(sup_l || sup_r);
   const bool left = sup_l || (!sup_r && ss > 0.0f);
-  float u[6], fx[6], Us[6];
   const PState<float, NV> K = pick_state(left, L, Rt);
-  float sk = left ? sl : sr, uk = left ? u_l : u_r;
-  p_uflux_f32<NV, CART>(K, g, dir, u, fx);
-  float iden = frcp(sk - ss);
-  Us[0] = K.rho * (sk - uk) * iden;
-  Us[1] = (u[1] * (sk - uk) - K.P * uk + p_s * ss) * iden;
-  float slr = sk * iscale;
+  const float sk = left ? sl : sr, uk = left ? u_l : u_r;
+  float vcov[3], vsq = 0.0f;
   for (int d = 0; d < NV; d++) {
-    float vs = (d == dir) ? ss * iscale : K.v[d];
-    Us[2 + d] = (CART ? vs : g.gcov[d] * vs) * Us[0];
+    vcov[d] = CART ? K.v[d] : g.gcov[d] * K.v[d];
+    vsq += K.v[d] * vcov[d];
   }
-  for (int q = 0; q < 2 + NV; q++) flux[q] = star ? fx[q] + slr * (Us[q] - u[q]) : fx[q];
-  if (NS) flux[MDS_YI] = flux[0] * K.ye;     // passive scalar: upwind by the contact
+  const float vn = K.v[dir], etot = 0.5f * K.rho * vsq + K.uu;
+  const float iden = frcp(sk - ss);
+  const float rs = K.rho * (sk - uk) * iden;
+  const float es = (etot * (sk - uk) - K.P * uk + p_s * ss) * iden;
+  const float slr = sk * iscale, vs = ss * iscale;
+  const float f0 = K.rho * vn, f1 = vn * (etot + K.P), fn = f0 * vcov[dir] + K.P;
+  flux[0] = star ? f0 + slr * (rs - K.rho) : f0;
+  flux[1] = star ? f1 + slr * (es - etot) : f1;
+  flux[2 + dir] = star ? fn + slr * ((CART ? vs : g.gcov[dir] * vs) * rs - K.rho * vcov[dir]) : fn;
+  for (int d = 0; d < NV; d++)
+    if (d != dir) flux[2 + d] = flux[0] * vcov[d];
+  if (NS) flux[MDS_YI] = flux[0] * K.ye;
   return isshock;
 }
 
@@ -631,12 +640,13 @@ MDS_DEV void hlle_f32(const PState<float, NV> &L, const PState<float, NV> &Rt,
 #pragma clang fp contract(fast)
   float u_l = CART ? L.v[dir] : L.v[dir] * g.scale;
   float u_r = CART ? Rt.v[dir] : Rt.v[dir] * g.scale;
-  float cs_l = fsqrt(L.G * L.P * frcp(L.rho));
-  float cs_r = fsqrt(Rt.G * Rt.P * frcp(Rt.rho));
+  const float rs_l = frsqrt(L.rho), rs_r = frsqrt(Rt.rho);
+  float cs_l = fsqrt(L.G * L.P) * rs_l;
+  float cs_r = fsqrt(Rt.G * Rt.P) * rs_r;
   float sl, sr, ss, p_s;
   int isshock;
-  wave_speeds_f32<false, CART, UNIG>(L.rho, Rt.rho, L.P, Rt.P, L.G, Rt.G, u_l, u_r, cs_l, cs_r, sl, sr, ss, p_s,
-                                     isshock, gk);
+  wave_speeds_f32<CART, UNIG>(L.rho, Rt.rho, L.P, Rt.P, L.G, Rt.G, u_l, u_r, cs_l, cs_r, rs_l, rs_r, sl, sr, ss, p_s,
+                              isshock, gk);
   float ul[6], ur[6], fl[6], fr[6];
   p_uflux_f32<NV, CART, NS>(L, g, dir, ul, fl);
   p_uflux_f32<NV, CART, NS>(Rt, g, dir, ur, fr);

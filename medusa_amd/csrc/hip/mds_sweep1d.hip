@@ -804,6 +804,7 @@ MDS_DEV void stage_f32(const DevProb &pb, const DevEos &eos, const Geo32 (&g)[Z]
                        const double (&gz)[Z], const Roles (&r)[Z], Lim32 &lim, Prim<float> (&o)[Z])
 {
   const float gam = (float)pb.gam;
+  const GamF32 gk = gam_f32_uniform(gam);      // the gamma law's wave-speed factors (unused with a table)
   constexpr int NQ = TAB ? 5 + NV : 2 + NV;
   float press[Z], cs[Z], qv[Z][NQ];
   double dpress[Z];
@@ -857,7 +858,7 @@ MDS_DEV void stage_f32(const DevProb &pb, const DevEos &eos, const Geo32 (&g)[Z]
     }
     float Ff[6] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f}, sig = 1.0f;
     int isshock = 0;
-    if (g[k].area >= 1.0e-16) isshock = hllc_f32<NV, !SPH, TAB>(L, Rt, g[k].fg, 0, Ff, sig);
+    if (g[k].area >= 1.0e-16) isshock = hllc_f32<NV, !SPH, TAB, !TAB>(L, Rt, g[k].fg, 0, Ff, sig, &gk);
     else sig = 1.0e-30f;
     if (r[k].face) lim.rate = fmaxf(lim.rate, fabsf(sig) * (float)pb.idx[0]);
     lim.nsh += __popcll(__ballot(r[k].count && isshock));

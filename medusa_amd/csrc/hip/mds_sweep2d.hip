@@ -50,9 +50,7 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
   const R gam = (R)pb.gam;
   const R gm1 = (R)(pb.gam - 1.0);
   const R igm1 = (R)(1.0 / (pb.gam - 1.0));
-  // the wave-speed factors of Gamma are formed per face here (one set per
-  // launch measured 0.8% slower in FP32 on a 2048^2 Kelvin-Helmholtz box)
-  const GamSet gk{};
+  const GamSet gk = gam_set_uniform(pb.gam);   // the gamma law's wave-speed factors
   const double area0 = pb.area[0], area1 = pb.area[1];
   const StateArrays<R> &in = (stage == 0) ? sp : sph;
   const bool col_out = (lane >= 2) && (lane <= 61) && (i >= 0) && (i < n1);
@@ -111,7 +109,7 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
 
   R Fx[5], sx;
   int shx;
-  xsweep<R, NV, SLAB, false>(W[2], pextra_of(j0), rgx, gam, gk, igm1, area0, Fx, sx, shx);
+  xsweep<R, NV, SLAB>(W[2], pextra_of(j0), rgx, gam, gk, igm1, area0, Fx, sx, shx);
   if (xface_ok) smax_x = sx > smax_x ? sx : smax_x;
   if (xface_ok && lane < 62) nshock += shx;
   int tag_cur = zone_tag(shx) | stage1_tag(j0);
@@ -129,7 +127,7 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
     recon_cell<R, NV, SLAB>(W[1], W[2], W[3], rg, igm1, yl_cur, yr_cur);
     bool hl = (tag_prev | tag_cur) != 0;
     R sy;
-    solve<R, NV, false>(yr_prev, yl_cur, gam, gk, area1, 1, hl, Fym, sy);
+    solve<R, NV>(yr_prev, yl_cur, gam, gk, area1, 1, hl, Fym, sy);
     if (col_out) {
       smax_y = sy > smax_y ? sy : smax_y;
       if (j0 == 0) nhlle += hl;   // face j0 is also the last face of the chunk below
@@ -151,7 +149,7 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
     } else if (j + 1 < j1) {
       R F2[5], s2;
       int sh2;
-      xsweep<R, NV, SLAB, false>(W[3], pextra_of(j + 1), rgx, gam, gk, igm1, area0, F2, s2, sh2);
+      xsweep<R, NV, SLAB>(W[3], pextra_of(j + 1), rgx, gam, gk, igm1, area0, F2, s2, sh2);
       if (xface_ok) smax_x = s2 > smax_x ? s2 : smax_x;
       if (xface_ok && lane < 62) nshock += sh2;
       tag_next = zone_tag(sh2) | stage1_tag(j + 1);
@@ -167,7 +165,7 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
     }
     R Fyp[5], sy;
     bool hl = (tag_cur | tag_next) != 0;
-    solve<R, NV, false>(yr_cur, yl_next, gam, gk, area1, 1, hl, Fyp, sy);
+    solve<R, NV>(yr_cur, yl_next, gam, gk, area1, 1, hl, Fyp, sy);
     if (col_out) {
       smax_y = sy > smax_y ? sy : smax_y;
       nhlle += hl;

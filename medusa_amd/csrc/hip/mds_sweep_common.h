@@ -233,9 +233,8 @@ MDS_DEV void recon_cell(const Cell<R, NV> &m, const Cell<R, NV> &c, const Cell<R
 
 // Riemann solve in direction d; returns isshock.  FP64: area-weighted flux
 // in reference order.  FP32: flux per unit area (the FP64 accumulate applies
-// the area).  UNIG: the gamma law's wave-speed factors come from gk instead
-// of being formed per face.  |signal speed| returned in ssig.
-template <class R, int NV, bool UNIG = true>
+// the area).  The gamma law's wave-speed factors come from gk.  |signal speed| returned in ssig.
+template <class R, int NV>
 MDS_DEV int solve(const Cell<R, NV> &l, const Cell<R, NV> &r, R gam, const GamSet &gk, double area, int d,
                   bool use_hlle, R F[5], R &ssig)
 {
@@ -249,14 +248,14 @@ MDS_DEV int solve(const Cell<R, NV> &l, const Cell<R, NV> &r, R gam, const GamSe
   if constexpr (std::is_same<R, double>::value) {
     g.area = area;
     double s = 0.0;
-    if (use_hlle) hlle_x64<NV, true, 0, UNIG>(L, Rt, g, d, F, s, &gk.f64);
-    else sh = hllc_x64<NV, true, 0, UNIG>(L, Rt, g, d, F, s, &gk.f64);
+    if (use_hlle) hlle_x64<NV, true, 0, true>(L, Rt, g, d, F, s, &gk.f64);
+    else sh = hllc_x64<NV, true, 0, true>(L, Rt, g, d, F, s, &gk.f64);
     ssig = fabs(s);
   } else {
     g.area = 1.0f;
     float s = 0.0f;
-    if (use_hlle) hlle_f32<NV, true, 0, UNIG>(L, Rt, g, d, F, s, &gk.f32);
-    else sh = hllc_f32<NV, true, 0, UNIG>(L, Rt, g, d, F, s, &gk.f32);
+    if (use_hlle) hlle_f32<NV, true, 0, true>(L, Rt, g, d, F, s, &gk.f32);
+    else sh = hllc_f32<NV, true, 0, true>(L, Rt, g, d, F, s, &gk.f32);
     ssig = fabsf(s);
   }
   return sh;
@@ -265,7 +264,7 @@ MDS_DEV int solve(const Cell<R, NV> &l, const Cell<R, NV> &r, R gam, const GamSe
 // x sweep of one row: per-lane flux through the lower x face, its shock tag
 // and |signal speed|.  Lane 63 additionally needs P of the zone above it so
 // that the tag of its own face is exact (pextra).
-template <class R, int NV, bool SLAB = false, bool UNIG = true>
+template <class R, int NV, bool SLAB = false>
 MDS_DEV void xsweep(const Cell<R, NV> &me, R pextra, const typename ReconGeoT<R>::type &rgx, R gam,
                     const GamSet &gk, R igm1, double area, R F[5], R &ssig, int &isshock)
 {
@@ -287,7 +286,7 @@ MDS_DEV void xsweep(const Cell<R, NV> &me, R pextra, const typename ReconGeoT<R>
   L.uu = lane_from_below(ar.uu);
   for (int d = 0; d < NV; d++) L.v[d] = lane_from_below(ar.v[d]);
   L.P = lane_from_below(ar.P);
-  isshock = solve<R, NV, UNIG>(L, al, gam, gk, area, 0, false, F, ssig);
+  isshock = solve<R, NV>(L, al, gam, gk, area, 0, false, F, ssig);
 }
 
 // shock tags only (P reconstruction + the HLLC pressure-jump test, riemann.c:374-383)

@@ -505,3 +505,39 @@ def test_c4_size_columns_fp32_density_pressure_velocity():
         say(f"  column {k} n={g.n[0]}: L1 {err}; moving zones {int(moving.sum())}")
         assert err["rho"] <= FP32_RHO_TOL and err["p"] <= FP32_RHO_TOL
         assert err["v/cs"] <= FP32_RHO_TOL and err["v_moving"] <= 1e-3
+
+
+@pytest.mark.parametrize("sph", [False, True])
+@pytest.mark.parametrize("kind, dp, dv", [("near", 1.0e-3, 0.0), ("rarefaction", 0.2, 1.5), ("shock", 0.2, -1.5)])
+def test_fp32_tubes_in_each_branch_of_the_star_pressure(kind, dp, dv, sph):
+    """FP32-bulk tubes and columns of 130 zones (more than one segment of every
+    launch shape) against FP64, whose middle face starts in the
+    primitive-variable, the two-rarefaction or the two-shock star pressure.  A
+    step rounds the state to 2^-24 and the star pressure's power turns some ten
+    roundings of its argument into at most 80 eps; sixty steps of that at
+    random signs stay below 1e-5 of the L1 norms (velocities against the sound
+    speed)."""
+    n = 130
+    x0, x1 = (0.0, np.log(10.0)) if sph else (0.0, 1.0)
+    g = mds.GridBuilder(1, [n], [x0], [(x1 - x0) / n], geom=mds.GEOM_SPHERICAL if sph else mds.GEOM_CARTESIAN,
+                        rcoord=mds.RCOORD_LOG if sph else mds.RCOORD_UNIFORM)
+    prob = dict(grid=g, bc_lo=[mds.BC_OUTFLOW], bc_hi=[mds.BC_OUTFLOW], gam=1.4)
+    x = x0 + (np.arange(n) + 0.5) * (x1 - x0) / n
+    right = np.arange(n) >= n // 2
+    scale = np.exp(x) if sph else np.ones(n)                  # v^x = v_r / r on log r
+    p = np.zeros((5, 1, 1, n))
+    p[0, 0, 0] = 1.0 + 0.1 * right
+    p[1, 0, 0] = (1.0 + dp * right) / 0.4
+    p[2, 0, 0] = np.where(right, 0.5, -0.5) * dv / scale
+    out = []
+    for prec in (mds.FP64, mds.FP32_BULK):
+        ctx = mds.Context([prob], precision=prec, rp=mds.run_params(cfl=0.5))
+        ctx.upload(p)
+        ctx.update_eos()
+        ctx.run(60)
+        out.append(ctx.download()[:, 0, 0])
+    a, b = out[1], out[0]
+    errs = [np.sum(np.abs(a[k] - b[k])) / np.sum(np.abs(b[k])) for k in (0, 1)]
+    errs.append(np.sum(np.abs(a[2] - b[2]) * scale) / (n * np.sqrt(1.4)))
+    say(f"fp32 tube, {kind}, spherical={sph}: L1 rho, u, v/cs {errs}")
+    assert max(errs) <= 1.0e-5
