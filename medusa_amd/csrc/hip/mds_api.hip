@@ -1826,6 +1826,7 @@ __global__ void recon_points_x64(int n, const double *a, const double *mom, cons
   g.xlo = x[2 * c];
   g.xhi = x[2 * c + 1];
   recon_geo_x64(g);
+  g.y0 = drcp(g.g0);
   para_recon_x64(a[3 * c], a[3 * c + 1], a[3 * c + 2], g, al[c], ar[c]);
 }
 

@@ -311,6 +311,8 @@ MDS_DEV int face_flux(const DevProb &pb, int lev, int fd, double q[4][8], bool p
     gr.xhi = pb.startx[D] + ((fd + 1) * s) * pb.dx[D];
     recon_geo_x64(gl);
     recon_geo_x64(gr);
+    gl.y0 = drcp(gl.g0);
+    gr.y0 = drcp(gr.g0);
     gl.order = gr.order = pb.order;
     double Lq[8], Rq[8];
     if (polar) {
@@ -411,6 +413,7 @@ MDS_DEV void zone_recon(const DevProb &pb, int lev, int zd, const double q3[3][8
     g.xlo = pb.startx[D] + (zd * s) * pb.dx[D];
     g.xhi = pb.startx[D] + ((zd + 1) * s) * pb.dx[D];
     recon_geo_x64(g);
+    g.y0 = drcp(g.g0);
     g.order = pb.order;
 #pragma unroll
     for (int v = 0; v < 8; v++) {

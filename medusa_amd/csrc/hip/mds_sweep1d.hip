@@ -222,7 +222,7 @@ struct Geo64 {
   ReconGeo64 rg;
   FaceGeo<double> fg;
   const double *zg;         // zone record (spherical)
-  double vol;
+  double vol, yvol;         // zone volume and its reciprocal
   double gcov0[3], gcon[3];
 };
 
@@ -241,6 +241,7 @@ MDS_DEV void load_geo64(const DevProb &pb, int c, int n, Geo64 &g)
   rg.xlo = pb.startx[0] + c * pb.dx[0];
   rg.xhi = pb.startx[0] + (c + 1) * pb.dx[0];
   recon_geo_x64(rg);
+  rg.y0 = drcp(rg.g0);
   rg.order = pb.order;
   if (SPH) {
     const double *zg = pb.zone + (size_t)q * MDS_ZG_COUNT;
@@ -261,6 +262,7 @@ MDS_DEV void load_geo64(const DevProb &pb, int c, int n, Geo64 &g)
     g.vol = pb.volume;
     for (int d = 0; d < 3; d++) { g.gcov0[d] = 1.0; g.gcon[d] = 1.0; }
   }
+  g.yvol = drcp(g.vol);
 }
 
 // conserved form (fluid.c:4-25), Ye in slot MDS_YI
@@ -410,23 +412,23 @@ MDS_DEV Prim<double> stage_x64(const DevProb &pb, const DevEos &eos, const Geo64
   const double pf = stage == 0 ? 1.0 : 0.5, phf = stage == 0 ? 0.0 : 0.5, ff = stage == 0 ? 1.0 : 0.5;
   for (int k = 0; k < 2 + NV; k++) {
     double divF = (0.0 + Fp[k]) - F[k];
-    double ddt = (divF / g.vol) - src[k];
+    double ddt = div_y(divF, g.vol, g.yvol) - src[k];
     U[k] = ((pf * U[k]) + (phf * Uh[k])) - ((ff * dt) * ddt);
   }
   if (TAB) {
     const int k = MDS_YI;
     double divF = (0.0 + Fp[k]) - F[k];
-    double ddt = (divF / g.vol) - src[k];
+    double ddt = div_y(divF, g.vol, g.yvol) - src[k];
     U[k] = ((pf * U[k]) + (phf * Uh[k])) - ((ff * dt) * ddt);
   }
   u_to_p_x64<NV, !SPH>(U, g.gcon, o.rho, o.uu, o.v);
-  if (TAB) o.ye = U[MDS_YI] / U[0];
+  if (TAB) o.ye = div_x64(U[MDS_YI], U[0]);
   if (stage == 1) {
     // estimate_dt zone bound (step.c:177-187): new velocity, sound speed of
     // the eos array as last filled (from this stage's input state)
-    if (!TAB) cs = sqrt((gam * press) / q.rho);
+    if (!TAB) cs = sqrt_x64(div_x64(gam * press, q.rho));
     double sc0 = SPH ? zg[MDS_ZG_SCALE0] : 1.0;
-    double loc = (fabs(o.v[0]) + (SPH ? cs / sc0 : cs)) / pb.dx[0];
+    double loc = div_x64(fabs(o.v[0]) + (SPH ? div_x64(cs, sc0) : cs), pb.dx[0]);
     lim.locmax = fmax(lim.locmax, loc);
   }
   return o;

@@ -139,6 +139,8 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
   const double idx0 = 1.0 / pb.dx[0], idx1 = 1.0 / pb.dx[1];
   // the update's constants, read from the record once (see GeoDir)
   const double volume = pb.volume, gamd = pb.gam, dxs[3] = {pb.dx[0], pb.dx[1], pb.dx[2]};
+  const double yvol = uniform_f64(drcp(volume));
+  const double ydx[3] = {uniform_f64(drcp(dxs[0])), uniform_f64(drcp(dxs[1])), uniform_f64(drcp(dxs[2]))};
   const double g0[3] = {SRC ? pb.g0[0] : 0.0, SRC ? pb.g0[1] : 0.0, SRC ? pb.g0[2] : 0.0};
   for (int j = j0; j < j1; j++) {
     load_row(j + 2, W[4]);
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
       if constexpr (X64) {
         for (int q = 0; q < 2 + NV; q++) {
           double divF = ((((0.0 + Fxp_cur[q]) - Fxm_cur[q]) + Fyp[q]) - Fym[q]);
-          double ddt = (divF / volume) - src[q];
+          double ddt = div_y(divF, volume, yvol) - src[q];
           U[q] = ((pf * U[q]) + (phf * Uh[q])) - ((ff * dt) * ddt);
         }
         u_to_p_x64<NV, true>(U, one3, ro, uo, vo);
@@ -235,10 +237,10 @@ __global__ __launch_bounds__(256) void sweep2d(Sweep2DArgs a, StateArrays<R> sp,
       if (stage == 1) {
         double loc;
         if constexpr (X64) {
-          double cs = sqrt((gamd * press) / rho);
+          double cs = sqrt_x64(div_x64(gamd * press, rho));
           loc = 0.0;
-          loc += (fabs(vo[0]) + cs) / dxs[0];
-          loc += (fabs(NV > 1 ? vo[1] : 0.0) + cs) / dxs[1];
+          loc += div_y(fabs(vo[0]) + cs, dxs[0], ydx[0]);
+          loc += div_y(fabs(NV > 1 ? vo[1] : 0.0) + cs, dxs[1], ydx[1]);
         } else {
           float cs = fsqrt((float)gamd * (float)press * frcp((float)rho));
           loc = (fabs(vo[0]) + cs) * idx0 + (fabs(NV > 1 ? vo[1] : 0.0) + cs) * idx1;

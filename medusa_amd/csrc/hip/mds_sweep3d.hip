@@ -162,6 +162,8 @@ __global__ __launch_bounds__((TY + 4) * 64) void sweep3d(Sweep3DArgs a, StateArr
 
   // the update's constants, read from the record once (see GeoDir)
   const double volume = pb.volume, gamd = pb.gam, dxs[3] = {pb.dx[0], pb.dx[1], pb.dx[2]};
+  const double yvol = uniform_f64(drcp(volume));
+  const double ydx[3] = {uniform_f64(drcp(dxs[0])), uniform_f64(drcp(dxs[1])), uniform_f64(drcp(dxs[2]))};
   const double g0[3] = {SRC ? pb.g0[0] : 0.0, SRC ? pb.g0[1] : 0.0, SRC ? pb.g0[2] : 0.0};
   const double area[3] = {pb.area[0], pb.area[1], pb.area[2]};
   for (int k = k0; k < k1; k++) {
@@ -284,7 +286,7 @@ __global__ __launch_bounds__((TY + 4) * 64) void sweep3d(Sweep3DArgs a, StateArr
         for (int q = 0; q < 2 + NV; q++) {
           double divF = ((((0.0 + Fxp_cur[q]) - Fxm_cur[q]) + sFy[q][w + 1][lane]) - sFy[q][w][lane]);
           divF += Fzp[q] - Fzm[q];
-          double ddt = (divF / volume) - src[q];
+          double ddt = div_y(divF, volume, yvol) - src[q];
           U[q] = ((pf * U[q]) + (phf * Uh[q])) - ((ff * dt) * ddt);
         }
         u_to_p_x64<NV, true>(U, one3, ro, uo, vo);
@@ -312,9 +314,9 @@ __global__ __launch_bounds__((TY + 4) * 64) void sweep3d(Sweep3DArgs a, StateArr
       if (stage == 1) {
         double loc;
         if constexpr (X64) {
-          double cs = sqrt((gamd * press) / rho);
+          double cs = sqrt_x64(div_x64(gamd * press, rho));
           loc = 0.0;
-          for (int d = 0; d < 3; d++) loc += (fabs(d < NV ? vo[d] : 0.0) + cs) / dxs[d];
+          for (int d = 0; d < 3; d++) loc += div_y(fabs(d < NV ? vo[d] : 0.0) + cs, dxs[d], ydx[d]);
         } else {
           float cs = fsqrt((float)gamd * (float)press * frcp((float)rho));
           loc = 0.0;
@@ -508,6 +510,8 @@ __global__ __launch_bounds__(TY * 64) void sweep3dh(Sweep3DArgs a, StateArrays<R
 
   // the update's constants, read from the record once (see GeoDir)
   const double volume = pb.volume, gamd = pb.gam, dxs[3] = {pb.dx[0], pb.dx[1], pb.dx[2]};
+  const double yvol = uniform_f64(drcp(volume));
+  const double ydx[3] = {uniform_f64(drcp(dxs[0])), uniform_f64(drcp(dxs[1])), uniform_f64(drcp(dxs[2]))};
   const double g0[3] = {SRC ? pb.g0[0] : 0.0, SRC ? pb.g0[1] : 0.0, SRC ? pb.g0[2] : 0.0};
   const double area[3] = {pb.area[0], pb.area[1], pb.area[2]};
   for (int k = k0; k < k1; k++) {
@@ -656,7 +660,7 @@ __global__ __launch_bounds__(TY * 64) void sweep3dh(Sweep3DArgs a, StateArrays<R
         for (int q = 0; q < 2 + NV; q++) {
           double divF = ((((0.0 + Fxp_cur[q]) - Fxm_cur[q]) + sFy[q][r + 1][lane]) - sFy[q][r][lane]);
           divF += Fzp[q] - Fzm[q];
-          double ddt = (divF / volume) - src[q];
+          double ddt = div_y(divF, volume, yvol) - src[q];
           U[q] = ((pf * U[q]) + (phf * Uh[q])) - ((ff * dt) * ddt);
         }
         u_to_p_x64<NV, true>(U, one3, ro, uo, vo);
@@ -684,9 +688,9 @@ __global__ __launch_bounds__(TY * 64) void sweep3dh(Sweep3DArgs a, StateArrays<R
       if (stage == 1) {
         double loc;
         if constexpr (X64) {
-          double cs = sqrt((gamd * press) / rho);
+          double cs = sqrt_x64(div_x64(gamd * press, rho));
           loc = 0.0;
-          for (int d = 0; d < 3; d++) loc += (fabs(d < NV ? vo[d] : 0.0) + cs) / dxs[d];
+          for (int d = 0; d < 3; d++) loc += div_y(fabs(d < NV ? vo[d] : 0.0) + cs, dxs[d], ydx[d]);
         } else {
           float cs = fsqrt((float)gamd * (float)press * frcp((float)rho));
           loc = 0.0;

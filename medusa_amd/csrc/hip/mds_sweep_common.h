@@ -56,7 +56,7 @@ template <class R>
 struct GeoDir {
   const double *mom, *rg;
   const float *rc;
-  double dx;
+  double dx, y0;           // zone width and (FP64) its reciprocal
   int qmax, order;
   MDS_DEV GeoDir(const DevProb &pb, int d)
   {
@@ -64,6 +64,7 @@ struct GeoDir {
     rg = pb.rg64[d];
     rc = pb.rc[d];
     dx = pb.dx[d];
+    y0 = std::is_same<R, double>::value ? uniform_f64(drcp(dx)) : 0.0;
     qmax = pb.n[d] + 2 * MDS_NG - 2;
     order = pb.order;
   }
@@ -84,6 +85,7 @@ MDS_DEV void load_rgeo(const GeoDir<R> &G, int z, typename ReconGeoT<R>::type &g
     g.a0 = m[3]; g.b0 = m[4];
     g.ap = m[6]; g.bp = m[7];
     g.gm = g.g0 = g.gp = G.dx;
+    g.y0 = G.y0;
     g.den = t[MDS_RG_DEN]; g.den2 = t[MDS_RG_DEN2];
     g.xlo = t[MDS_RG_XLO]; g.xhi = t[MDS_RG_XHI];
     g.order = G.order;
@@ -301,7 +303,7 @@ MDS_DEV int xshock_only(R P, R pextra, const typename ReconGeoT<R>::type &rgx)
   else recon<R>(qm, P, qp, rgx, al, ar);
   R p_l = lane_from_below(ar), p_r = al;
   R p_max = p_l > p_r ? p_l : p_r, p_min = p_l > p_r ? p_r : p_l;
-  if constexpr (std::is_same<R, double>::value) return ((p_max - p_min) / p_min > 0.5) ? 1 : 0;
+  if constexpr (std::is_same<R, double>::value) return (p_min >= 0.0 && (p_max - p_min) > 0.5 * p_min) ? 1 : 0;   // see wave_speeds_x64
   else return ((p_max - p_min) > 0.5f * p_min) ? 1 : 0;
 }
 

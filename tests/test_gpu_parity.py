@@ -541,3 +541,45 @@ def test_fp32_tubes_in_each_branch_of_the_star_pressure(kind, dp, dv, sph):
     errs.append(np.sum(np.abs(a[2] - b[2]) * scale) / (n * np.sqrt(1.4)))
     say(f"fp32 tube, {kind}, spherical={sph}: L1 rho, u, v/cs {errs}")
     assert max(errs) <= 1.0e-5
+
+
+@pytest.mark.parametrize("solver", [0, 1])
+def test_fp64_riemann_at_the_branch_points_matches_oracle(solver):
+    """Pressure ratios exactly at, one double below and one above the shock
+    flag's 3/2 and the star pressure's 2 (which the device decides on products
+    instead of quotients), equal sides, a vacuum side and denominators with
+    full mantissas: the flags equal the oracle's, the fluxes to a few
+    roundings."""
+    base = np.array([1.0, 1.0 / 3.0, 0.1, 7.0e27, 3.3e-11])
+    ratio = [1.0, 1.5, 2.0]
+    rows = []
+    for b in base:
+        for q in ratio:
+            for step in (-1, 0, 1):
+                p = b * q
+                p = p if step == 0 else np.nextafter(p, np.inf if step > 0 else 0.0)
+                for swap in (False, True):
+                    for du in (0.0, 1.0e-3, -1.0e-3, 0.4, -0.4):
+                        rows.append((p, b, du) if swap else (b, p, du))
+    rows += [(0.0, 1.0, 0.0), (1.0, 0.0, 0.0)]
+    n = len(rows)
+    pl, pr = np.zeros((n, 7)), np.zeros((n, 7))
+    for k, (a, b, du) in enumerate(rows):
+        c = np.sqrt(max(a, b))                  # densities near 1: speeds near sqrt(p)
+        for st, pp, sg in ((pl, a, -0.5), (pr, b, 0.5)):
+            st[k, 0] = 1.0 + 0.1 * (k % 7)
+            st[k, 1] = pp / 0.4
+            st[k, 2:5] = [sg * du * c, 0.3 * c, -0.2 * c]
+            st[k, 5] = pp
+            st[k, 6] = 1.4
+    fg = np.ones((n, 5))
+    f_gpu, s_gpu, sh_gpu = mds.riemann_points(mds.FP64, solver, pl, pr, fg, 0)
+    f_orc, s_orc, sh_orc = _oracle_riemann(solver, pl, pr, fg, 0)
+    assert np.array_equal(np.isnan(f_gpu).any(1), np.isnan(f_orc).any(1))
+    ok = ~np.isnan(f_orc).any(1)
+    scale = np.abs(f_orc[ok]).max(1, keepdims=True) + 1e-300
+    ferr = np.max(np.abs(f_gpu[ok] - f_orc[ok]) / scale)
+    say(f"riemann FP64 branch points solver={solver}: {n} faces, flux max rel {ferr:.3e}")
+    assert ferr < 1e-12 and np.max(np.abs(s_gpu[ok] - s_orc[ok]) / np.abs(s_orc[ok])) < 1e-12
+    if solver == 0:
+        assert np.array_equal(sh_gpu[ok], sh_orc[ok])
