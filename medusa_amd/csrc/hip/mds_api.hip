@@ -12,6 +12,7 @@
 #include <algorithm>
 #include "mds_internal.h"
 #include "mds_physics.h"
+#include "mds_clock.h"
 #include "mds_eos.h"
 #include "../../../include/mds_eos.h"
 #include "../common/mds_mp.h"
@@ -62,6 +63,8 @@ struct mds_ctx {
   Sph3Launch s3{};                 // its work buffers
   DevProb *dprob = nullptr;
   DevClock *dclock = nullptr;
+  DevClock *dclock2 = nullptr;     // 1D two-stage: second clocks and running minima of folded steps (mds_clock.h)
+  unsigned long long *dmind = nullptr;
   int2 *dseg = nullptr;            // 1D segment table of the single-stage kernels
   int nseg = 0;
   int2 *dseg2 = nullptr;           // 1D segment table of the two-stage kernel
@@ -93,14 +96,15 @@ struct mds_ctx {
   std::vector<double *> tdep_buf;                 // [prob][3 dirs][2 sides][2 stages], or null
   int ntdep = 0;
   std::vector<int> hdj, hdk;            // dendritic grid: dj and dk with ghosts (the grid's layout)
-  hipGraph_t graph[2] = {nullptr, nullptr};        // one step, per buffer parity
-  hipGraphExec_t gexec[2] = {nullptr, nullptr};
+  // one step, per buffer parity, then groups of folded steps, per parity
+  hipGraph_t graph[4] = {nullptr, nullptr, nullptr, nullptr};
+  hipGraphExec_t gexec[4] = {nullptr, nullptr, nullptr, nullptr};
   char err[512] = {0};
 };
 
 static void drop_graphs(mds_ctx *c)
 {
-  for (int k = 0; k < 2; k++) {
+  for (int k = 0; k < 4; k++) {
     if (c->gexec[k]) { hipGraphExecDestroy(c->gexec[k]); c->gexec[k] = nullptr; }
     if (c->graph[k]) { hipGraphDestroy(c->graph[k]); c->graph[k] = nullptr; }
   }
@@ -128,33 +132,13 @@ static int set_err(mds_ctx *c, int code, const char *fmt, ...)
 // small device kernels
 // ---------------------------------------------------------------------------
 
-// estimate_dt tail + dt policy (step.c:192-198, main.c:206-251), one thread
-// per problem.  The clock is advanced here (t += dt, istep++: main.c:263-264)
-// since the stage kernels only read dt.
+// the dt policy (mds_clock.h), one thread per problem
 __global__ void dt_policy_kernel(DevClock *ck, int nprob, RunParams rp)
 {
   int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nprob) return;
   DevClock c = ck[p];
-  if (!c.active) return;
-  if (!(c.t < c.tmax)) { ck[p].active = 0; return; }
-  double md = __longlong_as_double((long long)c.mindt);
-  if (c.istep == 0) md = (md < rp.initial_dt) ? md : rp.initial_dt;
-  md = (md < rp.dtmax) ? md : rp.dtmax;
-  md *= rp.cfl;
-  double dt = md;
-  if (dt < rp.dtmin) { ck[p].status = 1; ck[p].active = 0; return; }
-  if (c.istep == 0) dt *= rp.dt_init_safety;
-  else { double g = c.dtold * rp.dt_grow_safety; dt = (g < dt) ? g : dt; }
-  c.dtold = dt;
-  if (c.t + 1 * dt > c.tmax) dt = (1.000000001 * (c.tmax - c.t)) / 1;
-  if (dt < rp.dtmin) dt = rp.dtmin;
-  c.dt = dt;
-  // the reference's second-stage fill adds dt to the global t and takes it
-  // off again (bc.c:717-721, 1417), then the main loop adds dt (main.c:263)
-  c.t = ((c.t + dt) - dt) + dt;
-  c.istep += 1;
-  c.mindt = dt_key(1.0e100);   // step() resets min_dt (step.c:49)
+  if (dt_policy(c, __longlong_as_double((long long)c.mindt), rp)) c.mindt = dt_key(1.0e100);   // step() resets min_dt (step.c:49)
   ck[p] = c;
 }
 
@@ -333,6 +317,8 @@ extern "C" int mds_destroy(mds_ctx *c)
   for (void *g : c->geo_allocs) hipFree(g);
   if (c->dprob) hipFree(c->dprob);
   if (c->dclock) hipFree(c->dclock);
+  if (c->dclock2) hipFree(c->dclock2);
+  if (c->dmind) hipFree(c->dmind);
   if (c->dseg) hipFree(c->dseg);
   if (c->dseg2) hipFree(c->dseg2);
   if (c->dseg3) hipFree(c->dseg3);
@@ -902,6 +888,17 @@ static int create_impl(mds_ctx *c, const mds_problem *probs, int nprob, const md
     for (int p = 0; p < nprob; p++)
       if (c->hprob[p].bc_lo[0] == MDS_BC_PERIODIC || c->hprob[p].bc_hi[0] == MDS_BC_PERIODIC) c->can_fuse1d = 0;
     c->fuse1d = c->can_fuse1d;
+    // second clocks and running minima of folded steps (mds_clock.h)
+    if (c->can_fuse1d) {
+      const double big = 1.0e100;
+      unsigned long long k;
+      memcpy(&k, &big, sizeof(k));
+      const std::vector<unsigned long long> mind((size_t)nprob * MDS_FOLD, k);
+      HIPCHK(c, hipMalloc(&c->dclock2, sizeof(DevClock) * nprob));
+      HIPCHK(c, hipMemset(c->dclock2, 0, sizeof(DevClock) * nprob));
+      HIPCHK(c, hipMalloc(&c->dmind, sizeof(unsigned long long) * mind.size()));
+      HIPCHK(c, hipMemcpy(c->dmind, mind.data(), sizeof(unsigned long long) * mind.size(), hipMemcpyHostToDevice));
+    }
   } else {
     HIPCHK(c, hipMalloc(&c->dflags, (size_t)c->nzone));
     HIPCHK(c, hipMemset(c->dflags, 0, (size_t)c->nzone));
@@ -1117,6 +1114,9 @@ static int enqueue_stage(mds_ctx *c, int stage, int fp32)
   if (c->ndim == 1) {
     Sweep1DArgs a;
     a.zpl = 1;
+    a.fold = -1;
+    a.clock2 = nullptr;
+    a.mind = nullptr;
     a.seg = c->dseg;
     a.nseg = c->nseg;
     a.prob = c->dprob;
@@ -1194,9 +1194,12 @@ static int enqueue_stage(mds_ctx *c, int stage, int fp32)
 }
 
 // both RK stages of every 1D problem in one launch: p -> ph (the caller swaps)
-static int enqueue_fused1d(mds_ctx *c)
+static int enqueue_fused1d(mds_ctx *c, int fold = -1)
 {
   Sweep1DArgs a;
+  a.fold = fold;
+  a.clock2 = c->dclock2;
+  a.mind = c->dmind;
   a.zpl = c->fuse1d == 2 ? 2 : 1;
   a.seg = a.zpl == 2 ? c->dseg3 : c->dseg2;
   a.nseg = a.zpl == 2 ? c->nseg3 : c->nseg2;
@@ -1256,6 +1259,33 @@ static int enqueue_step(mds_ctx *c)
   return rc;
 }
 
+// Whether this context's two-stage steps run folded: a batch whose wavefronts
+// the device holds at once (16 per compute unit) waits for its steps' launches,
+// not for issue slots.  There the dt launch costs more than the policy in
+// every wavefront (a tube of 3001 zones in FP32 16.0 us a step with it, 6.8
+// folded and replayed; 820 wavefronts of FP64 columns 17.5 and 16.5 us); with
+// several rounds of wavefronts the policy costs more (1024 columns 115.0 and
+// 116.6 us, 300 rotating ones 49.1 and 50.1 us).
+static bool folds(const mds_ctx *c)
+{
+  return c->fuse1d && (c->fuse1d == 2 ? c->nseg3 : c->nseg2) <= 16 * std::max(1, c->ncu);
+}
+
+// A group of MDS_FOLD two-stage column steps without a dt launch between them
+// (mds_clock.h); the buffers' names end as they began.
+static int enqueue_group(mds_ctx *c)
+{
+  for (int f = 0; f < MDS_FOLD; f++) {
+    const int rc = enqueue_fused1d(c, f);
+    if (rc) {
+      if (f & 1) finish_step(c);          // the names of the last whole pair of steps
+      return rc;
+    }
+    finish_step(c);
+  }
+  return MDS_OK;
+}
+
 // One step of a context with time-dependent PROB hooks: the dt policy on
 // the device and a wait for it, the hooks on the host at the times the
 // reference's fills see (t and t + dt, bc.c:717-721), and their values
@@ -1296,6 +1326,8 @@ static int step_tdep(mds_ctx *c)
   return MDS_OK;
 }
 
+#define MDS_GRAPH_GROUPS 4     // groups of folded steps in one graph
+
 extern "C" int mds_run(mds_ctx *c, int nsteps)
 {
   if (!c || nsteps < 0) return MDS_EINVAL;
@@ -1306,7 +1338,12 @@ extern "C" int mds_run(mds_ctx *c, int nsteps)
     }
     return MDS_OK;
   }
-  for (int s = 0; s < nsteps; s++) {
+  int s = 0;
+  for (; folds(c) && s + MDS_FOLD <= nsteps; s += MDS_FOLD) {
+    int rc = enqueue_group(c);
+    if (rc) return rc;
+  }
+  for (; s < nsteps; s++) {
     int rc = enqueue_step(c);
     if (rc) return rc;
   }
@@ -1317,12 +1354,11 @@ extern "C" int mds_run_graph(mds_ctx *c, int nsteps)
 {
   if (!c || nsteps < 0) return MDS_EINVAL;
   if (c->ntdep > 0) return mds_run(c, nsteps);     // host hooks between the stages: no graph
-  for (int s = 0; s < nsteps; s++) {
-    // one graph per buffer parity: the two-stage 1D step alternates p and ph
-    const int k = c->fuse1d ? c->par : 0;
+  // launch graph k, captured first if it is new
+  auto replay = [&](int k, auto enqueue) -> int {
     if (!c->gexec[k]) {
       HIPCHK(c, hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
-      int rc = enqueue_step_kernels(c);
+      int rc = enqueue();
       hipGraph_t g = nullptr;
       hipError_t e = hipStreamEndCapture(c->st, &g);
       if (rc) { if (g) hipGraphDestroy(g); return rc; }
@@ -1331,6 +1367,27 @@ extern "C" int mds_run_graph(mds_ctx *c, int nsteps)
       HIPCHK(c, hipGraphInstantiate(&c->gexec[k], c->graph[k], nullptr, nullptr, 0));
     }
     HIPCHK(c, hipGraphLaunch(c->gexec[k], c->st));
+    return MDS_OK;
+  };
+  // one graph per buffer parity: the two-stage 1D step alternates p and ph.
+  // A launch of a graph takes the host some 16 us whatever it holds, which
+  // is a whole step of a small batch: folded steps replay MDS_GRAPH_GROUPS
+  // groups at a time.
+  const int par = c->fuse1d ? c->par : 0;
+  int s = 0;
+  for (; folds(c) && s + MDS_FOLD * MDS_GRAPH_GROUPS <= nsteps; s += MDS_FOLD * MDS_GRAPH_GROUPS) {
+    int rc = replay(2 + par, [&]() -> int {
+      for (int g = 0; g < MDS_GRAPH_GROUPS; g++) {
+        const int r1 = enqueue_group(c);
+        if (r1) return r1;
+      }
+      return MDS_OK;
+    });
+    if (rc) return rc;
+  }
+  for (; s < nsteps; s++) {
+    int rc = replay(c->fuse1d ? c->par : 0, [&]() -> int { return enqueue_step_kernels(c); });
+    if (rc) return rc;
     finish_step(c);
   }
   return MDS_OK;

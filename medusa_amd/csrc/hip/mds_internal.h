@@ -161,6 +161,11 @@ struct DevClock {
   unsigned long long nbad, noff;
 };
 
+// Which step of a group of MDS_FOLD consecutive steps a two-stage column
+// launch is: its wavefronts then apply the dt policy themselves (mds_clock.h)
+// instead of waiting for a launch of their own between the steps.
+#define MDS_FOLD 4
+
 struct RunParams {
   double cfl, dt_init_safety, dt_grow_safety, dtmin, dtmax, initial_dt;
 };
@@ -183,6 +188,9 @@ struct Sweep1DArgs {
   int persist;             // 1: persistent grid (resident workgroups walk the segment table)
   int gen;                 // the general instances: PROB/EXTRAP ghost layers, hydro_interp_order < 3
   int zpl;                 // two-stage FP32-bulk kernel: zones per lane (1 or 2)
+  int fold;                // two-stage kernels: step of its group (0 .. MDS_FOLD - 1), or -1: dt_policy_kernel ran
+  DevClock *clock2;        // the groups' second clocks and running minima (mds_clock.h)
+  unsigned long long *mind;
 };
 
 struct Sweep2DArgs {

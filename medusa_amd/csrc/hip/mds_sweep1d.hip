@@ -35,6 +35,7 @@
 #include "mds_physics.h"
 #include "mds_eos.h"
 #include "mds_gravity.h"
+#include "mds_clock.h"
 
 namespace {
 
@@ -100,8 +101,9 @@ struct Roles {
   bool own;     // the zone is owned by this wave (health counts)
 };
 
-// Fold the wave's limits into the problem clock (lane 0 of the wave).
-MDS_DEV void commit_limits(const DevProb &pb, DevClock *ck, unsigned long long *counters, int lane,
+// Fold the wave's limits into the problem's running minimum and clock (lane 0 of the wave).
+MDS_DEV void commit_limits(const DevProb &pb, DevClock *ck, unsigned long long *mindt, unsigned long long *counters,
+                           int lane,
                            const Lim1D &lim)
 {
   double wsmax = wave_max(lim.smax), wloc = wave_max(lim.locmax);
@@ -112,7 +114,7 @@ MDS_DEV void commit_limits(const DevProb &pb, DevClock *ck, unsigned long long *
     if (wloc > 0.0) l = fmin(l, 1.0 / wloc);
     if (wsrc < 1.0e300) l = fmin(l, wsrc / (0.0 + 1.0e-16));
     l = fmin(l, wlim);
-    if (l < 1.0e300) atomicMin(&ck->mindt, dt_key(l));
+    if (l < 1.0e300) atomicMin(mindt, dt_key(l));
     if (lim.nsh) atomicAdd(&counters[0], (unsigned long long)lim.nsh);
     if (lim.nbad) atomicAdd(&ck->nbad, (unsigned long long)lim.nbad);
     if (lim.noff) atomicAdd(&ck->noff, (unsigned long long)lim.noff);
@@ -483,12 +485,12 @@ __global__ __launch_bounds__(256) void sweep1d_x64(Sweep1DArgs a, StateArrays<do
       StateArrays<double> &out = (stage == 0) ? sph : sp;
       store_prims<NV, TAB>(out, off, c, o);
     }
-    commit_limits(pb, ck, a.counters, lane, lim);
+    commit_limits(pb, ck, &ck->mindt, a.counters, lane, lim);
   }
 }
 
 // FP64 two-stage kernel: reads in (U^n), writes out (U^{n+1}).
-template <int NV, bool SPH, int TAB>
+template <int NV, bool SPH, int TAB, bool FOLD>
 __global__ __launch_bounds__(256) void sweep1d2_x64(Sweep1DArgs a, StateArrays<double> in,
                                                     StateArrays<double> out)
 {
@@ -502,17 +504,18 @@ __global__ __launch_bounds__(256) void sweep1d2_x64(Sweep1DArgs a, StateArrays<d
     const int2 sg = a.seg[w];
     const DevProb &pb = a.prob[sg.x];
     DevClock *ck = &a.clock[sg.x];
+    const StepClock sc = step_clock<FOLD>(a, sg.x, sg.y == 0);
     const int n = pb.n[0];
     const int c0 = sg.y;
     const int c = c0 - 2 * MDS_NG + lane;
     const long long off = pb.off;
     const bool own = (lane >= 2 * MDS_NG) && (lane < 2 * MDS_NG + MDS_SEG1D2) && (c < n);
-    if (!ck->active) {
+    if (!sc.active) {
       // frozen problem: carry its state over to the output buffer
       if (own) store_prims<NV, TAB>(out, off, c, load_prims<NV, TAB>(in, off, c, 0));
       continue;
     }
-    const double dt = ck->dt;
+    const double dt = sc.dt;
     int flip;
     const int s = bc_src<false>(c, n, pb.bc_lo[0], pb.bc_hi[0], flip);
     const Prim<double> q = load_zone<NV, TAB, false>(pb, in, s, flip);
@@ -534,7 +537,7 @@ __global__ __launch_bounds__(256) void sweep1d2_x64(Sweep1DArgs a, StateArrays<d
     const Prim<double> o = stage_x64<NV, SPH, TAB, 0>(pb, a.eos, g, 1, dt, h, U0, q, 0.0, r1, lim);
     lim.nbad += bad_state_lanes(own, o.rho, o.uu, !TAB);
     if (own) store_prims<NV, TAB>(out, off, c, o);
-    commit_limits(pb, ck, a.counters, lane, lim);
+    commit_limits(pb, ck, sc.mindt, a.counters, lane, lim);
   }
 }
 
@@ -662,11 +665,12 @@ MDS_DEV float wave_min_f32(float v)
   return v;
 }
 
-MDS_DEV void commit_limits32(DevClock *ck, unsigned long long *counters, int lane, const Lim32 &lim)
+MDS_DEV void commit_limits32(DevClock *ck, unsigned long long *mindt, unsigned long long *counters, int lane,
+                             const Lim32 &lim)
 {
   const float w = wave_min_f32(fminf(frcp(lim.rate), lim.dts));
   if (lane == 0) {
-    if (w < __builtin_huge_valf()) atomicMin(&ck->mindt, dt_key((double)w));
+    if (w < __builtin_huge_valf()) atomicMin(mindt, dt_key((double)w));
     if (lim.nsh) atomicAdd(&counters[0], (unsigned long long)lim.nsh);
     if (lim.nbad) atomicAdd(&ck->nbad, (unsigned long long)lim.nbad);
     if (lim.noff) atomicAdd(&ck->noff, (unsigned long long)lim.noff);
@@ -936,14 +940,14 @@ __global__ __launch_bounds__(256) void sweep1d_f32(Sweep1DArgs a, StateArrays<fl
       StateArrays<float> &out = (stage == 0) ? sph : sp;
       store_prims<NV, TAB>(out, off, c, o[0]);
     }
-    commit_limits32(ck, a.counters, lane, lim);
+    commit_limits32(ck, &ck->mindt, a.counters, lane, lim);
   }
 }
 
 // Z zones per lane: the wave holds zones c0 - 4 + p, p = Z lane + k in
 // [0, 64 Z); stage 0 is valid for p in [2, 64 Z - 3], stage 1 for the owned
 // p in [4, 64 Z - 5] (64 Z - 8 zones per segment).
-template <int NV, bool SPH, int TAB, int Z>
+template <int NV, bool SPH, int TAB, int Z, bool FOLD>
 __global__ __launch_bounds__(256) void sweep1d2_f32(Sweep1DArgs a, StateArrays<float> in,
                                                     StateArrays<float> out)
 {
@@ -958,6 +962,7 @@ __global__ __launch_bounds__(256) void sweep1d2_f32(Sweep1DArgs a, StateArrays<f
     const int2 sg = a.seg[w];
     const DevProb &pb = a.prob[sg.x];
     DevClock *ck = &a.clock[sg.x];
+    const StepClock sc = step_clock<FOLD>(a, sg.x, sg.y == 0);
     const int n = pb.n[0];
     const int c0 = sg.y;
     const long long off = pb.off;
@@ -969,13 +974,13 @@ __global__ __launch_bounds__(256) void sweep1d2_f32(Sweep1DArgs a, StateArrays<f
       cz[k] = c0 - 2 * MDS_NG + p;
       own[k] = (p >= 2 * MDS_NG) && (p < 2 * MDS_NG + SEG) && (cz[k] < n);
     }
-    if (!ck->active) {
+    if (!sc.active) {
 #pragma unroll
       for (int k = 0; k < Z; k++)
         if (own[k]) store_prims<NV, TAB>(out, off, cz[k], load_prims<NV, TAB>(in, off, cz[k], 0));
       continue;
     }
-    const double dt = ck->dt;
+    const double dt = sc.dt;
     Prim<float> q[Z];
     Geo32 g[Z];
     double U0[Z][6];
@@ -1008,7 +1013,7 @@ __global__ __launch_bounds__(256) void sweep1d2_f32(Sweep1DArgs a, StateArrays<f
       lim.nbad += bad_state_lanes(own[k], o[k].rho, o[k].uu, !TAB);
       if (own[k]) store_prims<NV, TAB>(out, off, cz[k], o[k]);
     }
-    commit_limits32(ck, a.counters, lane, lim);
+    commit_limits32(ck, sc.mindt, a.counters, lane, lim);
   }
 }
 
@@ -1162,7 +1167,10 @@ extern "C" hipError_t mds_launch_sweep1d(int fp32, int nv, int sph, int tab, int
 #define MDS_L1G(K, ...) do { MDS_GRID((K<__VA_ARGS__>)) hipLaunchKernelGGL((K<__VA_ARGS__>), grid, block, 0, st, *a, p, h, stage); } while (0)
 // the general instances (PROB/EXTRAP ghost layers, hydro_interp_order < 3)
 #define MDS_L1(K, ...) do { if (a->gen) MDS_L1G(K, __VA_ARGS__, 1); else MDS_L1G(K, __VA_ARGS__, 0); } while (0)
-#define MDS_L2(K, ...) do { MDS_GRID((K<__VA_ARGS__>)) hipLaunchKernelGGL((K<__VA_ARGS__>), grid, block, 0, st, *a, p, h); } while (0)
+#define MDS_L2F(K, ...) do { MDS_GRID((K<__VA_ARGS__>)) hipLaunchKernelGGL((K<__VA_ARGS__>), grid, block, 0, st, *a, p, h); } while (0)
+// steps of a folded group have instances of their own: the policy's registers
+// cost the others 2% (300 rotating columns in FP32, 49.2 and 50.2 us)
+#define MDS_L2(K, ...) do { if (a->fold >= 0) MDS_L2F(K, __VA_ARGS__, true); else MDS_L2F(K, __VA_ARGS__, false); } while (0)
   if (!fp32) {
     const StateArrays<double> &p = *(const StateArrays<double> *)sp;
     const StateArrays<double> &h = *(const StateArrays<double> *)sph_;
@@ -1214,6 +1222,7 @@ extern "C" hipError_t mds_launch_sweep1d(int fp32, int nv, int sph, int tab, int
 #undef MDS_L1
 #undef MDS_L1G
 #undef MDS_L2
+#undef MDS_L2F
 #undef MDS_GRID
   return hipGetLastError();
 }

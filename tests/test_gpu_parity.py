@@ -583,3 +583,38 @@ def test_fp64_riemann_at_the_branch_points_matches_oracle(solver):
     assert ferr < 1e-12 and np.max(np.abs(s_gpu[ok] - s_orc[ok]) / np.abs(s_orc[ok])) < 1e-12
     if solver == 0:
         assert np.array_equal(sh_gpu[ok], sh_orc[ok])
+
+
+@pytest.mark.parametrize("precision", [mds.FP64, mds.FP32_BULK])
+@pytest.mark.parametrize("nsteps", [1, 3, 4, 5, 16, 23])
+@pytest.mark.parametrize("graph", [False, True])
+def test_folded_steps_match_single_steps(precision, nsteps, graph):
+    """Groups of four steps whose wavefronts apply the dt policy themselves
+    (small batches) against the same steps taken one call at a time, which
+    launch the policy: the same bits and clocks, at step counts around the
+    groups' and the graphs' sizes, for columns of one, two and many segments
+    of which one stops at tmax inside a group."""
+    probs, states = [], []
+    for n, scale in ((40, 1.0), (130, 2.0), (700, 0.5)):
+        g = mds.GridBuilder(1, [n], [0.0], [1.0 / n])
+        probs.append(dict(grid=g, bc_lo=[mds.BC_OUTFLOW], bc_hi=[mds.BC_REFLECT], gam=1.4))
+        p = mds.init_sod(g)
+        p[1] *= scale
+        states.append(p)
+    out = []
+    for one_by_one in (True, False):
+        # the coarsest column reaches tmax after some ten steps (dt grows by 1.1)
+        ctx = mds.Context(probs, precision=precision, rp=mds.run_params(cfl=0.5, tmax=0.012))
+        for k, p in enumerate(states):
+            ctx.upload(p, k)
+        ctx.update_eos()
+        if one_by_one:
+            for _ in range(2 * nsteps):
+                ctx.run(1)
+        else:
+            ctx.run(nsteps, graph=graph)
+            ctx.run(nsteps, graph=graph)
+        out.append([(ctx.download(k), ctx.clock(k), ctx.health(k)) for k in range(3)])
+    for (a, ca, ha), (b, cb, hb) in zip(*out):
+        assert np.array_equal(a, b) and ca == cb and ha == hb
+    say(f"folded steps: 2 x {nsteps}, graph={graph}: clocks {[c[1] for c in out[1]]}")
