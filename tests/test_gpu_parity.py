@@ -618,3 +618,26 @@ def test_folded_steps_match_single_steps(precision, nsteps, graph):
     for (a, ca, ha), (b, cb, hb) in zip(*out):
         assert np.array_equal(a, b) and ca == cb and ha == hb
     say(f"folded steps: 2 x {nsteps}, graph={graph}: clocks {[c[1] for c in out[1]]}")
+
+
+@pytest.mark.parametrize("precision", [mds.FP64, mds.FP32_BULK])
+@pytest.mark.parametrize("n", [(7, 5), (456, 459), (457, 459), (1024, 1024), (1025, 1024), (1461, 1437)])
+def test_download_returns_what_was_uploaded(precision, n):
+    """States that come back in one piece or in several, at the sizes where
+    that changes (8 MB of all variables, 2^20 doubles and 2^21 floats of one),
+    exactly; with fewer variables than the context holds, with more (zeros),
+    and into memory that held other values."""
+    g = mds.GridBuilder(2, list(n), [0.0, 0.0], [1.0 / n[0], 1.0 / n[1]])
+    prob = dict(grid=g, bc_lo=[3, 3], bc_hi=[3, 3], gam=1.4)
+    r = np.random.default_rng(5)
+    p = np.zeros((5, 1, n[1], n[0]))
+    p[:4, 0] = r.uniform(0.5, 1.5, (4, n[1], n[0]))         # two velocity components
+    ctx = mds.Context([prob], precision=precision)
+    ctx.upload(p)
+    want = p if precision == mds.FP64 else p.astype(np.float32).astype(np.float64)
+    assert np.array_equal(ctx.download(), want)
+    for nvars in (2, 3, 7):
+        a = np.full((nvars, 1, n[1], n[0]), 7.0)
+        assert mds.lib().mds_download_prims(ctx.h, 0, a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), nvars) == 0
+        m = min(nvars, 5)
+        assert np.array_equal(a[:m], want[:m]) and not a[m:].any()
