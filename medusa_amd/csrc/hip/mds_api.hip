@@ -1447,7 +1447,9 @@ extern "C" int mds_run_graph(mds_ctx *c, int nsteps)
   auto replay = [&](int k, auto enqueue) -> int {
     if (!c->gexec[k]) {
       HIPCHK(c, hipStreamBeginCapture(c->st, hipStreamCaptureModeThreadLocal));
+      c->s3.serial = 1;
       int rc = enqueue();
+      c->s3.serial = 0;
       hipGraph_t g = nullptr;
       hipError_t e = hipStreamEndCapture(c->st, &g);
       if (rc) { if (g) hipGraphDestroy(g); return rc; }

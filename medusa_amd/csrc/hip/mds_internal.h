@@ -255,6 +255,7 @@ struct Sph3Launch {
   int mpl;                 // multipole gravity: lmax (0 = none)
   MpDev mp;
   int upd;                 // update workgroup shape (MDS_TILE_UPD3S)
+  int serial;              // the stage in one chain, without the second stream
 };
 
 #define MDS_SHELL_ROWS 32  // (j, k) rows per wavefront in the 3D shell-mass pass

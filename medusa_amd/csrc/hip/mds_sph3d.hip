@@ -639,15 +639,18 @@ __global__ void sph3_reset_flags(unsigned char *flags, long long n)
   if (z < n) flags[z] = 1;
 }
 
+// reset: the first stage's kernel also resets the step's tags.  A workgroup
+// takes 64 radial zones of four theta rows, so a zone's indices need no
+// division.
 template <class R>
-__global__ __launch_bounds__(256) void sph3_eos_kernel(Sph3Args a, StateArrays<R> in)
+__global__ __launch_bounds__(256) void sph3_eos_kernel(Sph3Args a, StateArrays<R> in, int reset)
 {
   const DevProb &pb = a.pb;
-  const long long nz = (long long)pb.n[0] * pb.n[1] * pb.n[2];
-  const long long z = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (z >= nz) return;
-  if (pb.lj && !dend_valid(pb, (int)(z % pb.n[0]), (int)((z / pb.n[0]) % pb.n[1]), (int)(z / ((long long)pb.n[0] * pb.n[1]))))
-    return;
+  const int i = blockIdx.x * 64 + (threadIdx.x & 63), j = blockIdx.y * 4 + (threadIdx.x >> 6), k = blockIdx.z;
+  if (i >= pb.n[0] || j >= pb.n[1]) return;
+  const long long z = zid3(pb, i, j, k);
+  if (reset) a.flags[z] = 1;
+  if (pb.lj && !dend_valid(pb, i, j, k)) return;
   double press, lt;
   int jt = a.tg[z];                    // the bracket search starts from the last one
   if (sizeof(R) == 8) {
@@ -1652,7 +1655,13 @@ __global__ __launch_bounds__(256, 3) void sph3_update(Sph3Args a, StateArrays<R>
 // ([e] records, {e} waits).  The shell masses read only rho; the listed
 // level-change faces need the EOS arrays, and the theta ones the radial shock
 // tags of both radial kernels; the update needs everything.  Both streams
-// have the default priority.
+// have the default priority.  In a context's own graphs (L.serial) the stage
+// is one chain instead: a graph's branches land on queues of their own that
+// wait some 10 us for each other, and six such waits a stage are more than
+// the overlap gives (a step of the dendritic star as a graph, forked and in
+// one chain: 160 x 32 x 64 FP64 559 and 515 us, 320 x 64 x 128 FP32 1000 and
+// 924 us, 640 x 128 x 256 6045 and 5968 us; eager, forked is the faster:
+// 466 and 499 us for the first).
 template <class R, int DEND>
 static hipError_t launch_stage(const Sph3Launch &L, const Sph3Args &a, const StateArrays<R> &sp,
                                const StateArrays<R> &sph, int stage, hipStream_t st)
@@ -1662,16 +1671,18 @@ static hipError_t launch_stage(const Sph3Launch &L, const Sph3Args &a, const Sta
   const long long nz = (long long)pb.n[0] * pb.n[1] * pb.n[2];
   const dim3 blk(256);
   const bool irr = DEND && (L.nirr[0] > 0 || L.nirr[1] > 0);
-  const bool fork = L.mono || irr;
+  const bool fork = (L.mono || irr) && !L.serial;
   hipStream_t s2 = fork ? L.side : st;
   hipError_t e = hipSuccess;
   auto rec = [&](int k, hipStream_t s) { if (fork && e == hipSuccess) e = hipEventRecord(L.ev[k], s); };
   auto wait = [&](hipStream_t s, int k) { if (fork && e == hipSuccess) e = hipStreamWaitEvent(s, L.ev[k], 0); };
   rec(0, st);
   wait(s2, 0);
-  if (stage == 0)
+  if (L.tab)
+    hipLaunchKernelGGL(sph3_eos_kernel<R>, dim3((unsigned)((pb.n[0] + 63) / 64), (unsigned)((pb.n[1] + 3) / 4), (unsigned)pb.n[2]),
+                       blk, 0, st, a, in, stage == 0);
+  else if (stage == 0)
     hipLaunchKernelGGL(sph3_reset_flags, dim3((unsigned)((nz + 255) / 256)), blk, 0, st, L.flags, nz);
-  if (L.tab) hipLaunchKernelGGL(sph3_eos_kernel<R>, dim3((unsigned)((nz + 255) / 256)), blk, 0, st, a, in);
   const dim3 pgrid((unsigned)((pb.n[0] + 63) / 64), (unsigned)L.npart);
   if (L.mono == MDS_MONOPOLE_GR) {
     // the pressure sums read the table EOS arrays of this stage: after the
