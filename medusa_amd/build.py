@@ -6,8 +6,9 @@
            program in the shape of the reference main loop, linked to libmds.so
 
 FP64 kernels are compiled with -ffp-contract=off so they round exactly like
-the reference CPU build; the FP32-bulk functions re-enable contraction locally
-with `#pragma clang fp contract(fast)`.  Packed FP32 instructions are disabled
+the reference CPU build; the FP32-bulk functions re-enable contraction within
+an expression with `#pragma clang fp contract(on)`: the source then decides
+which products are fused, and every kernel rounds alike.  Packed FP32 instructions are disabled
 (-packed-fp32-ops).
 
 Usage:  python -m medusa_amd.build   (or medusa_amd.build.build())

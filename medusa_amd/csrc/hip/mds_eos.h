@@ -164,7 +164,7 @@ MDS_DEV void eos_fill_x64(const DevEos &t, double rho, double u, double ye, doub
 // FP32-bulk interpolation: increments over the first corner in FP32
 MDS_DEV float eos_tri_f32(const float *rec, const EosW &w, int jt, double dtemp, float &base)
 {
-#pragma clang fp contract(fast)
+#pragma clang fp contract(on)
   const int jtp = jt + 1;
   const float a = (float)(1.0 - dtemp), b = (float)dtemp;
   const float c0 = (float)w.c0, c1 = (float)w.c1, c2 = (float)w.c2, c3 = (float)w.c3;

@@ -641,3 +641,30 @@ def test_download_returns_what_was_uploaded(precision, n):
         assert mds.lib().mds_download_prims(ctx.h, 0, a.ctypes.data_as(ctypes.POINTER(ctypes.c_double)), nvars) == 0
         m = min(nvars, 5)
         assert np.array_equal(a[:m], want[:m]) and not a[m:].any()
+
+
+@pytest.mark.parametrize("precision", [mds.FP64, mds.FP32_BULK])
+@pytest.mark.parametrize("n", [(5, 4, 4), (61, 9, 8), (20, 20, 20)])
+def test_random_boxes_have_the_same_bits_in_every_tile_shape(precision, n):
+    """3D boxes of random states, whose faces take every branch of the limiter
+    and the star pressure, in the tile shapes with and without halo wavefronts:
+    the kernels round alike."""
+    g = mds.GridBuilder(3, list(n), [0.0] * 3, [1.0 / 64] * 3)
+    prob = dict(grid=g, bc_lo=[mds.BC_OUTFLOW] * 3, bc_hi=[mds.BC_REFLECT] * 3, gam=1.4)
+    r = np.random.default_rng(11)
+    p = np.zeros((5,) + n[::-1])
+    p[:2] = r.uniform(0.8, 1.2, (2,) + n[::-1])
+    p[2:] = r.uniform(-0.3, 0.3, (3,) + n[::-1])
+    want = None
+    for ty, kc, hs in ((4, 4, 0), (4, 1, 0), (8, 4, 0), (4, 4, 1), (4, 1, 1), (8, 4, 1), (12, 4, 1)):
+        ctx = mds.Context([prob], precision=precision, rp=mds.run_params(cfl=0.4))
+        ctx.set_tile(mds.TILE_TY3D, ty)
+        ctx.set_tile(mds.TILE_KC3D, kc)
+        ctx.set_tile(mds.TILE_HALO3D, hs)
+        ctx.upload(p)
+        ctx.update_eos()
+        ctx.run(7)
+        got = ctx.download()
+        want = got if want is None else want
+        assert np.array_equal(got, want), (ty, kc, hs)
+    say(f"random box {n}: every tile shape alike")
