@@ -444,6 +444,98 @@ static int build_multipole(mds_ctx *c, const mds_grid *g, int lmax, Sph3Launch &
   return e;
 }
 
+// ---------------------------------------------------------------------------
+// launch shapes
+// ---------------------------------------------------------------------------
+// A marching kernel's piece of `len` rows (planes) costs len + 2 of them (the
+// window's start), and a piece shares its compute unit's issue slots with the
+// others there: few long pieces leave units idle and latencies bare, many
+// short ones repeat their starts.  The costs below are relative times per row
+// (plane), read off sweeps over the pieces on one MI355X.
+
+static bool gen3d(const mds_ctx *c);
+
+// 2D, rows per wavefront.  A row of one wavefront per SIMD waits for its own
+// latencies, so the second costs little (FP32: 5.0, 7.4, 8.3 and 10.2 us for 1
+// to 4 wavefronts; FP64 19.6 and 29.8 us for 1 and 2); from there the work
+// counts.  With the fixed 24 rows of before a 300^2 box took 140 us a step in
+// FP32 where 2 rows take 36, 64^2 in FP64 471 and 49, 777 x 1003 in FP64 511
+// (8 rows, the best of the shapes tried: 298) and 270 at 7 rows.
+static double cost2d(const mds_ctx *c, int rows)
+{
+  static const double t32[4] = {1.96, 2.9, 3.25, 4.0}, t64[2] = {1.4, 2.13};
+  const int fp32 = c->precision == MDS_FP32_BULK, held = fp32 ? 4 : 2;
+  const DevProb &h = c->hprob[0];
+  const double w = (double)((h.n[0] + MDS_SEG1D - 1) / MDS_SEG1D) * ((h.n[1] + rows - 1) / rows);
+  const double r = w / (4.0 * std::max(1, c->ncu));
+  const double t = r <= held ? (fp32 ? t32 : t64)[std::max(0, (int)ceil(r) - 1)]
+                             : std::max(r + 0.3, held + 1.0);     // a second round of wavefronts
+  return (rows + 2) * t;
+}
+
+// 3D, planes per workgroup of a tile shape.  FP32 tiles of 4 rows without halo
+// wavefronts run three to a compute unit (12.7 us a plane for one, 17.3 for
+// three, then 5.4 us each); every other tile fills its unit.  The FP64 tiles
+// of 4 rows with halo wavefronts take 36 us a plane, those of 8 without 58,
+// which decides between the two on small boxes.
+static double cost3d(const mds_ctx *c, int ty, int kc, int hs)
+{
+  const int fp32 = c->precision == MDS_FP32_BULK;
+  const DevProb &h = c->hprob[0];
+  const double w = (double)((h.n[0] + MDS_SEG1D - 1) / MDS_SEG1D) * ((h.n[1] + ty - 1) / ty) * ((h.n[2] + kc - 1) / kc);
+  const double r = w / std::max(1, c->ncu);
+  if (fp32 && ty == 4 && hs)
+    return (kc + 2) * (r <= 3.0 ? 12.7 + 2.3 * std::max(0.0, r - 1.0) : std::max(22.0, 5.4 * (r + 0.8)));
+  return (kc + 2) * (ty == 4 ? 36.0 : 58.0) * (r <= 8.0 ? std::max(1.0, ceil(r)) : r + 0.5);
+}
+
+static const int rows2d[] = {1, 2, 3, 4, 5, 6, 7, 8, 10, 12, 14, 16, 18, 20, 24, 32, 48, 64};
+static const int planes3d[] = {1, 2, 3, 4, 6, 8, 12, 16, 24, 32, 48, 64};
+
+// The cheapest rows per wavefront.
+static int rows_for(const mds_ctx *c)
+{
+  int best = 1;
+  for (int v : rows2d)
+    if (v <= c->hprob[0].n[1] && cost2d(c, v) < cost2d(c, best)) best = v;
+  return best;
+}
+
+// The cheapest planes per workgroup of a tile shape.
+static int planes_for(const mds_ctx *c, int ty, int hs)
+{
+  int best = 1;
+  for (int kc : planes3d)
+    if (kc <= c->hprob[0].n[2] && cost3d(c, ty, kc, hs) < cost3d(c, ty, best, hs)) best = kc;
+  return best;
+}
+
+// The shapes of a new context.  Boxes: the cheapest by the costs above; FP32
+// boxes in tiles of 4 rows without halo wavefronts, the fastest at every size
+// (256^3: 1.93 ms a step against 2.1 to 3.7 for the others; 150 x 122 x 203:
+// 0.50 ms, 0.87 with the fixed shape of before), FP64 boxes in the cheaper of
+// 4 rows with and 8 without (24^3: 77 us, 622 before; 256^3: 11.4 ms, 13.3).
+// FP32 columns: two zones per lane once one zone per lane is more wavefronts
+// than the device holds (1024 columns: 107 us against 143; below that the
+// wavefronts' latency counts, which one zone per lane has less of).
+static void default_shapes(mds_ctx *c)
+{
+  if (c->sph3) return;
+  if (c->ndim == 1) {
+    if (c->fuse1d && c->precision == MDS_FP32_BULK && c->nseg2 > 16 * std::max(1, c->ncu)) c->fuse1d = 2;
+  } else if (c->ndim == 2) {
+    c->chunk2d = rows_for(c);
+  } else {
+    c->ty3d = 4;
+    c->halo3d = c->precision == MDS_FP32_BULK && !gen3d(c);
+    c->kc3d = planes_for(c, c->ty3d, c->halo3d);
+    if (c->precision != MDS_FP32_BULK && !gen3d(c)) {
+      const int kc = planes_for(c, 8, 1);
+      if (cost3d(c, 8, kc, 1) < cost3d(c, 4, c->kc3d, 0)) { c->ty3d = 8; c->halo3d = 1; c->kc3d = kc; }
+    }
+  }
+}
+
 static int create_impl(mds_ctx *c, const mds_problem *probs, int nprob, const mds_run_params *rp)
 {
   c->nprob = nprob;
@@ -780,8 +872,6 @@ static int create_impl(mds_ctx *c, const mds_problem *probs, int nprob, const md
     }
   }
   c->nzone = c->zstart[nprob];
-  if (const char *e = getenv("MDS_TILE_ROWS2D")) c->chunk2d = atoi(e) > 0 ? atoi(e) : c->chunk2d;
-  if (c->ndim == 3 && c->hprob[0].n[2] < c->kc3d) c->kc3d = c->hprob[0].n[2];
   size_t rs = rsize(c);
   for (int k = 0; k < c->nstate; k++) {
     HIPCHK(c, hipMalloc(&c->p[k], (size_t)c->nzone * rs));
@@ -911,6 +1001,8 @@ static int create_impl(mds_ctx *c, const mds_problem *probs, int nprob, const md
     HIPCHK(c, hipMalloc(&c->dflags, (size_t)c->nzone));
     HIPCHK(c, hipMemset(c->dflags, 0, (size_t)c->nzone));
   }
+  default_shapes(c);
+  if (const char *e = getenv("MDS_TILE_ROWS2D")) c->chunk2d = atoi(e) > 0 ? atoi(e) : c->chunk2d;
   return MDS_OK;
 }
 
@@ -1788,15 +1880,19 @@ extern "C" int mds_autotune(mds_ctx *c, int nsteps, double *best_ms)
       if (c->can_fuse1d && c->precision == MDS_FP32_BULK) cand.push_back({2, g, 0});
     }
   } else if (c->ndim == 2) {
-    for (int v : {4, 6, 8, 12, 16, 24, 32, 48, 64})
-      if (v <= c->hprob[0].n[1]) cand.push_back({v, 0, 0});
+    // the rows whose cost is near the least
+    for (int v : rows2d)
+      if (v <= c->hprob[0].n[1] && cost2d(c, v) <= 1.15 * cost2d(c, rows_for(c))) cand.push_back({v, 0, 0});
   } else {
     // problems with PROB/EXTRAP ghost layers have one tile shape (4 rows,
     // halo wavefronts); only the planes per workgroup vary
     for (int hs : {0, 1})
-      for (int ty : {4, 8, 12})
-        for (int kc : {8, 16, 32, 64})
-          if (kc <= c->hprob[0].n[2] && (!gen3d(c) || (ty == 4 && hs == 0))) cand.push_back({ty, kc, hs});
+      for (int ty : {4, 8, 12}) {
+        if (gen3d(c) && (ty != 4 || hs)) continue;
+        const double least = cost3d(c, ty, planes_for(c, ty, hs), hs);
+        for (int kc : planes3d)
+          if (kc <= c->hprob[0].n[2] && cost3d(c, ty, kc, hs) <= 1.15 * least) cand.push_back({ty, kc, hs});
+      }
   }
   auto apply = [&](const Shape &v) {
     if (c->sph3) c->s3.upd = v.a;
@@ -1816,15 +1912,18 @@ extern "C" int mds_autotune(mds_ctx *c, int nsteps, double *best_ms)
     apply(v);
     double ms[3];
     rc = mds_run_timed(c, 1, ms);      // warm the shape
-    // best of two timed runs from the same state: one run of a few steps is
-    // at the mercy of clock ramps and other work on the device
+    // best of two timed runs from the same state, each of half a millisecond at
+    // least: one run of a few steps is at the mercy of clock ramps and other
+    // work on the device
+    int n = nsteps;
+    while (rc == MDS_OK && n * ms[0] < 0.5 && n < 64) n *= 2;
     double t = 1e300;
     for (int rep = 0; rep < 2 && rc == MDS_OK; rep++) {
       rc = snap_copy(c, s, false);
-      if (rc == MDS_OK) rc = mds_run_timed(c, nsteps, ms);
+      if (rc == MDS_OK) rc = mds_run_timed(c, n, ms);
       if (rc == MDS_OK && ms[0] < t) t = ms[0];
     }
-    if (rc == MDS_OK && t / nsteps < bms) { bms = t / nsteps; best = v; }
+    if (rc == MDS_OK && t / n < bms) { bms = t / n; best = v; }
     if (rc == MDS_OK) rc = snap_copy(c, s, false);
   }
   snap_free(s);

@@ -668,3 +668,49 @@ def test_random_boxes_have_the_same_bits_in_every_tile_shape(precision, n):
         want = got if want is None else want
         assert np.array_equal(got, want), (ty, kc, hs)
     say(f"random box {n}: every tile shape alike")
+
+
+@pytest.mark.parametrize("precision", [mds.FP64, mds.FP32_BULK])
+@pytest.mark.parametrize("n", [(4, 4), (61, 64), (129, 200), (5, 4, 4), (61, 9, 8), (70, 33, 37)])
+def test_default_launch_shapes_give_the_bits_of_fixed_ones(precision, n):
+    """The launch shape that a context takes from its sizes, for boxes around
+    the tiles' edges and smaller than one tile, against a fixed shape of long
+    pieces: the same bits and clocks, and pieces no longer than the box."""
+    nd = len(n)
+    g = mds.GridBuilder(nd, list(n), [0.0] * nd, [1.0 / 64] * nd)
+    prob = dict(grid=g, bc_lo=[mds.BC_OUTFLOW] * 3, bc_hi=[mds.BC_REFLECT] * 3, gam=1.4)
+    r = np.random.default_rng(11)
+    shape = tuple(n[::-1]) if nd == 3 else (1,) + tuple(n[::-1])
+    p = np.zeros((5,) + shape)
+    p[:2] = r.uniform(0.8, 1.2, (2,) + shape)
+    p[2:2 + nd] = r.uniform(-0.3, 0.3, (nd,) + shape)
+    out = []
+    for fixed in (False, True):
+        ctx = mds.Context([prob], precision=precision, rp=mds.run_params(cfl=0.4))
+        rows, planes = ctx.get_tile(mds.TILE_ROWS2D), ctx.get_tile(mds.TILE_KC3D)
+        if fixed and nd == 2:
+            ctx.set_tile(mds.TILE_ROWS2D, 24)
+        elif fixed:
+            ctx.set_tile(mds.TILE_TY3D, 4)
+            ctx.set_tile(mds.TILE_KC3D, 16)
+            ctx.set_tile(mds.TILE_HALO3D, 0)
+        else:
+            assert 1 <= (rows if nd == 2 else planes) <= n[-1]
+        ctx.upload(p)
+        ctx.update_eos()
+        ctx.run(7)
+        out.append((ctx.download(), ctx.clock(0)))
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+    say(f"default launch shape {n}: rows {rows}, planes {planes}")
+
+
+def test_default_shape_of_columns_by_their_number():
+    """FP32 columns take two zones per lane once one zone per lane is more than
+    16 wavefronts to a compute unit (4096 on the 256 units of an MI355X), FP64
+    ones never."""
+    n = 4096
+    g = mds.GridBuilder(1, [40], [0.0], [1.0 / 40])
+    prob = dict(grid=g, bc_lo=[mds.BC_OUTFLOW], bc_hi=[mds.BC_OUTFLOW], gam=1.4)
+    for count, precision, want in ((n // 2, mds.FP32_BULK, 1), (2 * n, mds.FP32_BULK, 2), (2 * n, mds.FP64, 1)):
+        ctx = mds.Context([prob] * count, precision=precision)
+        assert ctx.get_tile(mds.TILE_FUSE1D) == want
