@@ -1183,8 +1183,11 @@ static int pin_ready(mds_ctx *c)
 // widens and writes fresh memory at some 5 GB/s, so a state that fits the
 // staging comes over with one kernel that writes its variables there, and a
 // larger one in pieces, each of which the host's threads take out while the
-// next is on its way.  300 columns of 3000 zones with five variables: 16.8 ms
-// before, 6.7 now; 1024 columns 37 and 21.6 ms, 256^3 in FP32 122 and 15.5 ms.
+// next is on its way.  The kernel takes the pieces over too: the copy engine is
+// no faster, and its first use in a context costs 2 ms (the first 512^2 FP64
+// state 4.3 ms, 1.9 without it, 0.5 from then on).  300 columns of 3000 zones
+// with five variables: 16.8 ms before, 6.7 now; 1024 columns 37 and 21.6 ms,
+// 256^3 in FP32 122 and 15.5 ms.
 extern "C" int mds_download_prims(mds_ctx *c, int prob, double *prims, int nvars)
 {
   if (!c || prob < 0 || prob >= c->nprob || !prims || nvars < 2) return MDS_EINVAL;
@@ -1201,13 +1204,14 @@ extern "C" int mds_download_prims(mds_ctx *c, int prob, double *prims, int nvars
     }
   const int rc = pin_ready(c);
   if (rc) return rc;
+  const auto fetch = [&](long long o, long long n, unsigned v, char *to) {
+    const dim3 g((unsigned)((n + 255) / 256)), b(256);
+    if (fp32) hipLaunchKernelGGL(pack_kernel<float>, g, b, 0, c->st, arrays<float>(c->p), o, n, v, (float *)to);
+    else hipLaunchKernelGGL(pack_kernel<double>, g, b, 0, c->st, arrays<double>(c->p), o, n, v, (double *)to);
+    return hipGetLastError();
+  };
   const bool whole = nhave * nz * (long long)rs <= c->pin_half;
-  if (whole) {
-    const dim3 g((unsigned)((nz + 255) / 256)), b(256);
-    if (fp32) hipLaunchKernelGGL(pack_kernel<float>, g, b, 0, c->st, arrays<float>(c->p), off, nz, vars, (float *)c->pin);
-    else hipLaunchKernelGGL(pack_kernel<double>, g, b, 0, c->st, arrays<double>(c->p), off, nz, vars, (double *)c->pin);
-    HIPCHK(c, hipGetLastError());
-  }
+  if (whole) HIPCHK(c, fetch(off, nz, vars, c->pin));
   // while the state is on its way
   for (int k = 0; k < nvars; k++)
     if (k >= 6 || !(vars >> k & 1)) memset(prims + (size_t)k * nz, 0, (size_t)nz * sizeof(double));
@@ -1229,8 +1233,7 @@ extern "C" int mds_download_prims(mds_ctx *c, int prob, double *prims, int nvars
     if (!(vars >> k & 1)) continue;
     for (long long q = 0; q < nz; q += piece) {
       const long long mn = std::min(piece, nz - q);
-      HIPCHK(c, hipMemcpyAsync(c->pin + h * c->pin_half, (const char *)c->p[k] + (off + q) * rs, (size_t)mn * rs,
-                               hipMemcpyDeviceToHost, c->st));
+      HIPCHK(c, fetch(off + q, mn, 1u << k, c->pin + h * c->pin_half));
       HIPCHK(c, hipEventRecord(c->pin_ev[h], c->st));
       if (dst) {
         HIPCHK(c, hipEventSynchronize(c->pin_ev[h ^ 1]));

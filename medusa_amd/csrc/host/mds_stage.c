@@ -9,7 +9,7 @@
 #include <string.h>
 #include "../common/mds_stage.h"
 
-#define STAGE_PIECE (1LL << 15)     /* values a thread takes at a time */
+#define STAGE_PIECE (1LL << 14)     /* values a thread takes at a time */
 #define STAGE_THREADS 8
 
 void mds_stage_out(double *d, const void *s, int fp32, long long n)
