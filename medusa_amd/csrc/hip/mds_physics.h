@@ -682,13 +682,19 @@ MDS_DEV int hllc_f32(const PState<float, NV> &L, const PState<float, NV> &Rt,
   }
   const float vn = K.v[dir], etot = 0.5f * K.rho * vsq + K.uu;
   const float iden = frcp(sk - ss);
-  const float rs = K.rho * (sk - uk) * iden;
-  const float es = (etot * (sk - uk) - K.P * uk + p_s * ss) * iden;
+  // the star state's differences from the upwind state, which vanish exactly
+  // where the gas rests: formed as rho (sk - uk) / (sk - ss) less rho, the
+  // rounding of the reciprocal was a mass flux of eps rho c in uniform gas,
+  // and spherical columns drifted by it
+  const float rel = (ss - uk) * iden;
+  const float dr = K.rho * rel;
+  const float de = etot * rel + (p_s * ss - K.P * uk) * iden;
   const float slr = sk * iscale, vs = ss * iscale;
   const float f0 = K.rho * vn, f1 = vn * (etot + K.P), fn = f0 * vcov[dir] + K.P;
-  flux[0] = star ? f0 + slr * (rs - K.rho) : f0;
-  flux[1] = star ? f1 + slr * (es - etot) : f1;
-  flux[2 + dir] = star ? fn + slr * ((CART ? vs : g.gcov[dir] * vs) * rs - K.rho * vcov[dir]) : fn;
+  const float dm = K.rho * (vs - vn) + vs * dr;
+  flux[0] = star ? f0 + slr * dr : f0;
+  flux[1] = star ? f1 + slr * de : f1;
+  flux[2 + dir] = star ? fn + slr * (CART ? dm : g.gcov[dir] * dm) : fn;
   for (int d = 0; d < NV; d++)
     if (d != dir) flux[2 + d] = flux[0] * vcov[d];
   if (NS) flux[MDS_YI] = flux[0] * K.ye;
